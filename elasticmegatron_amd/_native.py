@@ -172,8 +172,8 @@ def set_tuning(blocks_per_cu: int = 0, nontemporal: bool = True, xcd_remap: int 
     bounded binary search); ``persistent=True`` selects a persistent grid, which ``blocks_per_cu``
     and ``run`` shape.  ``xcd_remap`` gives each of the 8 XCDs one contiguous eighth of the chunks:
     1 (or True) in the persistent grid and for plans of at least 2^19 chunks, 2 always, 0 (or False)
-    never.  ``warm_tables``: with the chunk table, a short kernel reads it and the segment
-    descriptors just before each copy, so that a launch after unrelated work starts from cached
+    never.  ``warm_tables``: with the chunk table, the first workgroups of each copy launch
+    read it and the segment descriptors, so that a launch after unrelated work starts from cached
     tables."""
     t = Tuning(blocks_per_cu, 1 if nontemporal else 0, int(xcd_remap), run, 1 if persistent else 0, lanes,
                units, 1 if buffer_ops else 0, 1 if chunk_index else 0, 1 if warm_tables else 0)

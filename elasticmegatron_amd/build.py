@@ -19,6 +19,7 @@ LIB = os.path.join(CSRC, "libemrs.so")
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",  # leading kernel arguments arrive in scalar registers
     "-Wall", "-Wno-unused-command-line-argument",
 ]
 

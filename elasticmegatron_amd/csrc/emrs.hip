@@ -113,6 +113,13 @@ struct Bases {
 };
 static_assert(sizeof(Bases) <= 1024, "Bases travels in kernel arguments");
 
+// The same for plans of at most 8 buffers a side (every plan over arenas, and
+// the resolved segment table of a plan over more than kArgBuffers).
+constexpr uint32_t kFewBuffers = 8;
+struct FewBases {
+  char *p[kFewBuffers];
+};
+
 // Where a chunk's segment search starts and ends: chunk c lies in one of the
 // segments first[c >> shift] .. first[(c >> shift) + 1], so the search spans
 // a few dozen segments of the plan instead of all of them.  Travels in
@@ -327,8 +334,8 @@ __device__ __forceinline__ void dispatch_units(uint32_t ul, const DevSeg &s, con
 // Base address of buffer i: from the kernel-argument table, or (kTable) from
 // a device-memory table of pointers for plans with more buffers than fit in
 // kernel arguments.
-template <bool kTable>
-__device__ __forceinline__ char *base_of(const Bases &b, const uint64_t *tab, uint32_t i) {
+template <bool kTable, typename B>
+__device__ __forceinline__ char *base_of(const B &b, const uint64_t *tab, uint32_t i) {
   if constexpr (kTable) return reinterpret_cast<char *>(tab[i]);
   else return b.p[i];
 }
@@ -606,6 +613,93 @@ __device__ __forceinline__ void dispatch_chunk(uint32_t ul, const DevSeg &s, con
   }
 }
 
+// Units [u0, u0 + L * U) of segment s by a workgroup of L lanes.
+template <bool kNT, int L, int U>
+__device__ __forceinline__ void copy_piece(const DevSeg &s, const char *sb, char *db, char *ab, uint32_t u0,
+                                           uint32_t total) {
+  const uint32_t ops = s.ops(), ul = s.unit_log2();
+  if (__builtin_expect(ops == 0 && ul == 4, 1)) {  // most of every plan
+    copy_units<u32x4, kNT, false, false, false, L, U>(s, sb, db, ab, u0, total);
+  } else if (ops & 4) {  // duplicate to aux, with or without zero fill
+    if (ops & 2) dispatch_chunk<kNT, true, true, L, U>(ul, s, sb, db, ab, u0, total);
+    else dispatch_chunk<kNT, false, true, L, U>(ul, s, sb, db, ab, u0, total);
+  } else if (ops & 1) {  // with the bf16 image (fp32 only: 16- or 4-byte units), with or without zero fill
+    if (ops & 2) {
+      if (ul == 4) copy_units<u32x4, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
+      else copy_units<uint32_t, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
+    } else {
+      if (ul == 4) copy_units<u32x4, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
+      else copy_units<uint32_t, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
+    }
+  } else if (ops & 2) {
+    dispatch_chunk<kNT, true, false, L, U>(ul, s, sb, db, ab, u0, total);
+  } else {
+    dispatch_chunk<kNT, false, false, L, U>(ul, s, sb, db, ab, u0, total);
+  }
+}
+
+// copy_piece with every unit width through buffer instructions.
+template <bool kNT, int L, int U>
+__device__ __forceinline__ void copy_piece_buf(const DevSeg &s, const char *sb, char *db, char *ab, uint32_t u0,
+                                               uint32_t total) {
+  const uint32_t ops = s.ops(), ul = s.unit_log2();
+  if (ops & 4) {
+    if (ops & 2) dispatch_chunk_buf<kNT, true, true, L, U>(ul, s, sb, db, ab, u0, total);
+    else dispatch_chunk_buf<kNT, false, true, L, U>(ul, s, sb, db, ab, u0, total);
+  } else if (ops & 1) {  // with the bf16 image (fp32 only: 16- or 4-byte units)
+    if (ops & 2) {
+      if (ul == 4) copy_units_buf<u32x4, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
+      else copy_units_buf<uint32_t, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
+    } else {
+      if (ul == 4) copy_units_buf<u32x4, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
+      else copy_units_buf<uint32_t, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
+    }
+  } else if (ops & 2) {
+    dispatch_chunk_buf<kNT, true, false, L, U>(ul, s, sb, db, ab, u0, total);
+  } else {
+    dispatch_chunk_buf<kNT, false, false, L, U>(ul, s, sb, db, ab, u0, total);
+  }
+}
+
+// A descriptor in one scalar load of 64 bytes.  `p` is uniform over the wave
+// and the table is never written while a kernel reads it.
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ DevSeg load_seg(const DevSeg *p) {
+  const u32x16 v = *reinterpret_cast<const __attribute__((address_space(4))) u32x16 *>(reinterpret_cast<uintptr_t>(p));
+  DevSeg s;
+  __builtin_memcpy(&s, &v, sizeof s);
+  return s;
+}
+
+// Workgroup `w` of the pre-read of a plan's lookup tables (its chunk table,
+// then its segment descriptors): the first workgroups of a copy launch read
+// both once, with cached loads.  Every copy workgroup starts with a dependent
+// load from the chunk table: after unrelated work those loads miss every
+// cache, each workgroup waits on HBM before its first data load, and the
+// launch ran 4.5% slower than one straight after another copy (whose table
+// reads left the table in the memory-side cache).  Read here first, with every
+// load in flight at once, the tables are in that cache when the copy's
+// workgroups follow, which the hardware dispatches in order; nothing waits for
+// them.  The XOR only keeps the loads; nothing is stored.
+constexpr uint32_t kWarmUnits = 4;  // 16-byte units per lane
+template <int L>
+__device__ __forceinline__ void warm_tables(const uint32_t *chunk_seg, const DevSeg *segs, uint64_t n_chunks,
+                                            uint32_t n_segs, uint32_t w) {
+  // Whole 16-byte units of the chunk table: its last 1-3 words share a line with the ones before.
+  const uint64_t na = n_chunks / 4, nb = (uint64_t)n_segs * (sizeof(DevSeg) / sizeof(u32x4));
+  const u32x4 *a = reinterpret_cast<const u32x4 *>(chunk_seg), *b = reinterpret_cast<const u32x4 *>(segs);
+  uint32_t acc = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < kWarmUnits; ++j) {
+    const uint64_t i = ((uint64_t)w * kWarmUnits + j) * L + threadIdx.x;
+    if (i < na + nb) {
+      const u32x4 v = i < na ? a[i] : b[i - na];
+      acc ^= v.x ^ v.y ^ v.z ^ v.w;
+    }
+  }
+  asm volatile("" ::"v"(acc));
+}
+
 // One workgroup of L lanes per piece of L * U units of a chunk (the default
 // schedule: L = 64, U = 1, four 1 KB pieces per chunk).  A chunk of 256 units
 // holds 256 / (L * U) pieces; workgroup w takes piece w % that of chunk
@@ -633,10 +727,16 @@ __global__ __launch_bounds__(L) void copy_plan_kernel(const DevSeg *__restrict__
                                                       SegHint hint, Bases src, Bases dst,
                                                       const uint64_t *__restrict__ src_tab,
                                                       const uint64_t *__restrict__ dst_tab, uint64_t xcd_share,
-                                                      const uint32_t *__restrict__ chunk_seg) {
+                                                      const uint32_t *__restrict__ chunk_seg, uint32_t n_warm,
+                                                      uint32_t n_segs) {
   constexpr uint32_t kPieces = kChunkUnits / (L * U);  // pieces per chunk: 1, 2 or 4
   static_assert(kPieces * L * U == kChunkUnits, "a piece divides a chunk");
   uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  if (w < n_warm) {
+    warm_tables<L>(chunk_seg, segs, n_chunks, n_segs, (uint32_t)w);
+    return;
+  }
+  w -= n_warm;
   if (w < xcd_share * 8) w = (w & 7) * xcd_share + (w >> 3);
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;
@@ -660,62 +760,47 @@ __global__ __launch_bounds__(L) void copy_plan_kernel(const DevSeg *__restrict__
   const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
   char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
   char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
-  const uint32_t ops = s.ops(), ul = s.unit_log2();
-  if constexpr (kBuf) {  // every unit width through buffer instructions
-    if (ops & 4) {
-      if (ops & 2) dispatch_chunk_buf<kNT, true, true, L, U>(ul, s, sb, db, ab, u0, total);
-      else dispatch_chunk_buf<kNT, false, true, L, U>(ul, s, sb, db, ab, u0, total);
-    } else if (ops & 1) {  // with the bf16 image (fp32 only: 16- or 4-byte units)
-      if (ops & 2) {
-        if (ul == 4) copy_units_buf<u32x4, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
-        else copy_units_buf<uint32_t, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
-      } else {
-        if (ul == 4) copy_units_buf<u32x4, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
-        else copy_units_buf<uint32_t, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
-      }
-    } else if (ops & 2) {
-      dispatch_chunk_buf<kNT, true, false, L, U>(ul, s, sb, db, ab, u0, total);
-    } else {
-      dispatch_chunk_buf<kNT, false, false, L, U>(ul, s, sb, db, ab, u0, total);
-    }
-    return;
-  }
-  if (ops & 4) {  // duplicate to aux, with or without zero fill
-    if (ops & 2) dispatch_chunk<kNT, true, true, L, U>(ul, s, sb, db, ab, u0, total);
-    else dispatch_chunk<kNT, false, true, L, U>(ul, s, sb, db, ab, u0, total);
-  } else if (ops & 1) {  // with the bf16 image (fp32 only: 16- or 4-byte units), with or without zero fill
-    if (ops & 2) {
-      if (ul == 4) copy_units<u32x4, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
-      else copy_units<uint32_t, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
-    } else {
-      if (ul == 4) copy_units<u32x4, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
-      else copy_units<uint32_t, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
-    }
-  } else if (ops & 2) {
-    dispatch_chunk<kNT, true, false, L, U>(ul, s, sb, db, ab, u0, total);
-  } else {
-    dispatch_chunk<kNT, false, false, L, U>(ul, s, sb, db, ab, u0, total);
-  }
+  if constexpr (kBuf) copy_piece_buf<kNT, L, U>(s, sb, db, ab, u0, total);
+  else copy_piece<kNT, L, U>(s, sb, db, ab, u0, total);
 }
 
-// Reads a plan's lookup tables (its chunk table, then its segment
-// descriptors) once, with cached loads, just before the copy.  Every copy
-// workgroup starts with a dependent load from the chunk table: after
-// unrelated work those loads miss every cache, each workgroup waits on HBM
-// before its first data load, and the launch ran 4.5% slower than one
-// straight after another copy (whose table reads left the table in the
-// memory-side cache).  Read here first, at HBM speed and with every load in
-// flight at once, the tables are in that cache when the copy starts.  The
-// XOR only keeps the loads; nothing is stored.
-__global__ __launch_bounds__(256) void warm_tables_kernel(const u32x4 *__restrict__ a, uint64_t na,
-                                                          const u32x4 *__restrict__ b, uint64_t nb) {
-  const uint64_t stride = (uint64_t)gridDim.x * 256;
-  uint32_t acc = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < na + nb; i += stride) {
-    const u32x4 v = i < na ? a[i] : b[i - na];
-    acc ^= v.x ^ v.y ^ v.z ^ v.w;
+// copy_plan_kernel of the default launch: with the chunk table and 64-bit
+// global addresses.  A workgroup lives for its chain of dependent scalar loads
+// (arguments, chunk-table entry, descriptor, bases) and one round trip to HBM,
+// so the chain is kept short: the leading arguments arrive in scalar registers
+// (the build preloads 14 words of them), the descriptor is one 64-byte scalar
+// load, and plans of at most 8 buffers a side (every arena plan) carry only
+// those, 0.2 KB of arguments for the host to write per launch instead of 3 KB.
+// Against copy_plan_kernel after a separate launch that read the tables (one
+// process, same allocations, back to back / after a 512 MiB fill): 14.5 MB of
+// traffic 13.5 / 16.0 us -> 8.7 / 12.0, 113 MB 27.7 / 33.7 -> 24.0 / 29.6,
+// 1.0 GB 162 / 168 -> 157 / 162, 70 GB 10587 / 10594 -> 10549 / 10547.
+template <bool kNT, bool kTable, int L, int U, typename B>
+__global__ __launch_bounds__(L) void copy_pieces_kernel(const uint32_t *__restrict__ chunk_seg,
+                                                        const DevSeg *__restrict__ segs, uint64_t n_chunks,
+                                                        uint64_t xcd_share, uint32_t gx, uint32_t n_warm,
+                                                        const uint64_t *__restrict__ src_tab,
+                                                        const uint64_t *__restrict__ dst_tab, B src, B dst,
+                                                        uint32_t n_segs) {
+  constexpr uint32_t kPieces = kChunkUnits / (L * U);  // pieces per chunk: 1, 2 or 4
+  static_assert(kPieces * L * U == kChunkUnits, "a piece divides a chunk");
+  uint64_t w = (uint64_t)blockIdx.y * gx + blockIdx.x;
+  if (w < n_warm) {
+    warm_tables<L>(chunk_seg, segs, n_chunks, n_segs, (uint32_t)w);
+    return;
   }
-  asm volatile("" ::"v"(acc));
+  w -= n_warm;
+  if (w < xcd_share * 8) w = (w & 7) * xcd_share + (w >> 3);
+  const uint64_t c = w / kPieces;
+  if (c >= n_chunks) return;
+  const DevSeg s = load_seg(segs + chunk_seg[c]);
+  const uint32_t total = s.len * s.rows;
+  const uint32_t u0 = (uint32_t)(c - s.chunk_begin) * kChunkUnits + (uint32_t)(w % kPieces) * (L * U);
+  const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
+  char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
+  char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
+  if (kPieces > 1 && u0 >= total) return;
+  copy_piece<kNT, L, U>(s, sb, db, ab, u0, total);
 }
 
 // Writes the chunk table from the device segment table: segment k owns the
@@ -2076,40 +2161,75 @@ int emrs_plan_create(const emrs_segment *segs, uint64_t n_segs, const uint64_t *
 }  // extern "C"
 
 namespace {
+// One launch of the copy over every piece of a plan.
+struct CopyLaunch {
+  const ResolvedBases *rb;
+  const uint64_t *stab, *dtab;  // device pointer tables when rb->table
+  const DevSeg *table;
+  uint32_t n_segs, n_bufs;      // n_bufs: buffers on the larger side whose bases rb holds
+  uint64_t n_chunks;
+  const SegHint *hint;
+  const uint32_t *cseg;         // the chunk table, or nullptr: the kernel searches
+  bool nt, warm;
+  hipStream_t st;
+};
+
+template <bool kNT, bool kTable, int L, int U, bool kBuf>
+void launch_kernel(const CopyLaunch &c, dim3 grid, uint64_t xcd_share, uint32_t n_warm) {
+  if constexpr (!kBuf) {
+    if (c.cseg) {
+      if (c.n_bufs <= kFewBuffers || kTable) {
+        FewBases src{}, dst{};
+        for (uint32_t i = 0; i < kFewBuffers && !kTable; ++i) src.p[i] = c.rb->src.p[i], dst.p[i] = c.rb->dst.p[i];
+        hipLaunchKernelGGL((copy_pieces_kernel<kNT, kTable, L, U, FewBases>), grid, dim3(L), 0, c.st, c.cseg, c.table,
+                           c.n_chunks, xcd_share, grid.x, n_warm, c.stab, c.dtab, src, dst, c.n_segs);
+      } else if constexpr (!kTable) {
+        hipLaunchKernelGGL((copy_pieces_kernel<kNT, false, L, U, Bases>), grid, dim3(L), 0, c.st, c.cseg, c.table,
+                           c.n_chunks, xcd_share, grid.x, n_warm, c.stab, c.dtab, c.rb->src, c.rb->dst, c.n_segs);
+      }
+      return;
+    }
+  }
+  hipLaunchKernelGGL((copy_plan_kernel<kNT, kTable, L, U, kBuf>), grid, dim3(L), 0, c.st, c.table, c.n_chunks, *c.hint,
+                     c.rb->src, c.rb->dst, c.stab, c.dtab, xcd_share, c.cseg, n_warm, c.n_segs);
+}
+
 template <int L, int U, bool kBuf>
-void launch_chunks(bool nt, const ResolvedBases &rb, dim3 grid, hipStream_t st, const DevSeg *table,
-                   uint64_t n_chunks, const SegHint &hint, const uint64_t *stab, const uint64_t *dtab,
-                   const uint32_t *cseg) {
-  const dim3 block(L);
+int launch_chunks(const CopyLaunch &c) {
+  const uint64_t n_pieces = c.n_chunks * (kChunkUnits / (L * U));
   const uint32_t remap = g_tuning.xcd_remap.load();
-  const bool by_xcd = remap == 2 || (remap == 1 && n_chunks >= kXcdRemapMinChunks);
-  const uint64_t xcd_share = by_xcd ? n_chunks * (kChunkUnits / (L * U)) / 8 : 0;
-  if (nt && rb.table)
-    hipLaunchKernelGGL((copy_plan_kernel<true, true, L, U, kBuf>), grid, block, 0, st, table, n_chunks, hint,
-                       rb.src, rb.dst, stab, dtab, xcd_share, cseg);
-  else if (nt)
-    hipLaunchKernelGGL((copy_plan_kernel<true, false, L, U, kBuf>), grid, block, 0, st, table, n_chunks, hint,
-                       rb.src, rb.dst, stab, dtab, xcd_share, cseg);
-  else if (rb.table)
-    hipLaunchKernelGGL((copy_plan_kernel<false, true, L, U, kBuf>), grid, block, 0, st, table, n_chunks, hint,
-                       rb.src, rb.dst, stab, dtab, xcd_share, cseg);
-  else
-    hipLaunchKernelGGL((copy_plan_kernel<false, false, L, U, kBuf>), grid, block, 0, st, table, n_chunks, hint,
-                       rb.src, rb.dst, stab, dtab, xcd_share, cseg);
+  const bool by_xcd = remap == 2 || (remap == 1 && c.n_chunks >= kXcdRemapMinChunks);
+  const uint64_t xcd_share = by_xcd ? n_pieces / 8 : 0;
+  // Workgroups that read the tables first, a multiple of 8 so that the pieces keep their XCDs.
+  uint64_t n_warm = 0;
+  if (c.cseg && c.warm) {
+    const uint64_t units = c.n_chunks / 4 + (uint64_t)c.n_segs * (sizeof(DevSeg) / sizeof(u32x4));
+    n_warm = ((units + kWarmUnits * L - 1) / (kWarmUnits * L) + 7) / 8 * 8;
+    if (n_warm > 0xffffffffull) n_warm = 0;
+  }
+  // A grid of at most 65535 rows, each a multiple of 8 workgroups long when there are several.
+  const uint64_t n_wg = n_warm + n_pieces;
+  uint64_t gx = std::min<uint64_t>(n_wg, std::max<uint64_t>(1ull << 16, (n_wg + kMaxGridY - 1) / kMaxGridY));
+  if (gx < n_wg) gx = (gx + 7) / 8 * 8;
+  if (gx > 0xffffffffull / L) return fail(EMRS_ERR_INVALID_ARGUMENT, "plan has too many chunks for one launch");
+  const dim3 grid((uint32_t)gx, (uint32_t)((n_wg + gx - 1) / gx));
+  if (c.nt && c.rb->table) launch_kernel<true, true, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
+  else if (c.nt) launch_kernel<true, false, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
+  else if (c.rb->table) launch_kernel<false, true, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
+  else launch_kernel<false, false, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
+  return EMRS_OK;
 }
 
 // The one-workgroup-per-piece launch for `lanes` lanes of `units` units each.
 template <bool kBuf>
-void launch_pieces(uint32_t lanes, uint32_t units, bool nt, const ResolvedBases &rb, dim3 grid, hipStream_t st,
-                   const DevSeg *table, uint64_t n_chunks, const SegHint &hint, const uint64_t *stab,
-                   const uint64_t *dtab, const uint32_t *cseg) {
+int launch_pieces(uint32_t lanes, uint32_t units, const CopyLaunch &c) {
   switch (lanes * 8 + units) {
-    case 64 * 8 + 1: launch_chunks<64, 1, kBuf>(nt, rb, grid, st, table, n_chunks, hint, stab, dtab, cseg); break;
-    case 64 * 8 + 2: launch_chunks<64, 2, kBuf>(nt, rb, grid, st, table, n_chunks, hint, stab, dtab, cseg); break;
-    case 128 * 8 + 1: launch_chunks<128, 1, kBuf>(nt, rb, grid, st, table, n_chunks, hint, stab, dtab, cseg); break;
-    case 128 * 8 + 2: launch_chunks<128, 2, kBuf>(nt, rb, grid, st, table, n_chunks, hint, stab, dtab, cseg); break;
-    case 256 * 8 + 1: launch_chunks<256, 1, kBuf>(nt, rb, grid, st, table, n_chunks, hint, stab, dtab, cseg); break;
-    default: launch_chunks<64, 4, kBuf>(nt, rb, grid, st, table, n_chunks, hint, stab, dtab, cseg); break;
+    case 64 * 8 + 1: return launch_chunks<64, 1, kBuf>(c);
+    case 64 * 8 + 2: return launch_chunks<64, 2, kBuf>(c);
+    case 128 * 8 + 1: return launch_chunks<128, 1, kBuf>(c);
+    case 128 * 8 + 2: return launch_chunks<128, 2, kBuf>(c);
+    case 256 * 8 + 1: return launch_chunks<256, 1, kBuf>(c);
+    default: return launch_chunks<64, 4, kBuf>(c);
   }
 }
 }  // namespace
@@ -2162,12 +2282,8 @@ int emrs_plan_execute(emrs_plan *plan, void *const *src_bases, void *const *dst_
   const uint32_t nseg = (uint32_t)plan->segs.size();
   const dim3 block(kThreads);
   if (!g_tuning.persistent.load()) {
-    // One workgroup per piece of lanes * units units, on a grid of at most 65535 rows.
+    // One workgroup per piece of lanes * units units.
     const uint32_t lanes = g_tuning.lanes.load(), units = g_tuning.units.load();
-    const uint64_t n_wg = plan->n_chunks * (kChunkUnits / (lanes * units));
-    const uint64_t gx = std::min<uint64_t>(n_wg, std::max<uint64_t>(1ull << 16, (n_wg + kMaxGridY - 1) / kMaxGridY));
-    if (gx > 0xffffffffull / lanes) return fail(EMRS_ERR_INVALID_ARGUMENT, "plan has too many chunks for one launch");
-    const dim3 grid((uint32_t)gx, (uint32_t)((n_wg + gx - 1) / gx));
     uint64_t *tab = nullptr;
     bool tab_owned = false;
     rc = pointer_table(plan, dev, rb, st, &tab, &tab_owned);
@@ -2177,6 +2293,7 @@ int emrs_plan_execute(emrs_plan *plan, void *const *src_bases, void *const *dst_
     // table: no per-workgroup base lookup.
     const ResolvedBases *lb = &rb;
     ResolvedBases flat;
+    uint32_t n_bufs = std::max(plan->stats.n_src_bufs, plan->stats.n_dst_bufs);
     if (rb.table && !tab_owned) {
       DevSeg *abs = nullptr;
       char *common = nullptr;
@@ -2186,6 +2303,7 @@ int emrs_plan_execute(emrs_plan *plan, void *const *src_bases, void *const *dst_
         table = abs;
         flat.src.p[0] = flat.dst.p[0] = common;
         lb = &flat;
+        n_bufs = 1;
         stab = dtab = nullptr;
       }
     }
@@ -2197,18 +2315,13 @@ int emrs_plan_execute(emrs_plan *plan, void *const *src_bases, void *const *dst_
         return rc;
       }
     }
-    if (cseg && g_tuning.warm_tables.load()) {
-      // 16-byte loads over the whole chunk table (its last 1-3 words share a line with the ones
-      // before) and every segment descriptor.
-      const uint64_t na = plan->n_chunks / 4, nb = (uint64_t)nseg * sizeof(DevSeg) / sizeof(u32x4);
-      const uint64_t blocks = std::min<uint64_t>((na + nb + 255) / 256, 4096);
-      hipLaunchKernelGGL(warm_tables_kernel, dim3((uint32_t)blocks), dim3(256), 0, st,
-                         reinterpret_cast<const u32x4 *>(cseg), na, reinterpret_cast<const u32x4 *>(table), nb);
+    const CopyLaunch launch{lb, stab, dtab, table, nseg, n_bufs, plan->n_chunks, &plan->hint,
+                            cseg, nt, g_tuning.warm_tables.load() != 0, st};
+    rc = g_tuning.buffer_ops.load() ? launch_pieces<true>(lanes, units, launch) : launch_pieces<false>(lanes, units, launch);
+    if (rc) {
+      if (tab_owned) (void)hipFreeAsync(tab, st);
+      return rc;
     }
-    if (g_tuning.buffer_ops.load())
-      launch_pieces<true>(lanes, units, nt, *lb, grid, st, table, plan->n_chunks, plan->hint, stab, dtab, cseg);
-    else
-      launch_pieces<false>(lanes, units, nt, *lb, grid, st, table, plan->n_chunks, plan->hint, stab, dtab, cseg);
     hipError_t le = hipGetLastError();
     if (tab_owned) (void)hipFreeAsync(tab, st);
     if (le != hipSuccess) return hip_fail(le, "copy_plan_kernel launch");

@@ -159,8 +159,8 @@ int emrs_plan_stats_get(const emrs_plan *plan, emrs_plan_stats *out);
  * checked and may be NULL.  The first call on a device uploads the plan's
  * tables (segment table, chunk table and, beyond 128 buffers a side, its
  * pointer table for these bases) synchronously; later calls with the same bases enqueue the copy
- * kernel, preceded by the table pre-read of emrs_tuning.warm_tables, and
- * nothing else, so they may be captured into a HIP graph.  Calls with
+ * kernel (whose first workgroups do the table pre-read of
+ * emrs_tuning.warm_tables) and nothing else, so they may be captured into a HIP graph.  Calls with
  * other bases than the first beyond 128 buffers allocate a stream-ordered
  * pointer table.  Neither the first call nor such a call may be captured:
  * while `stream` is capturing they return EMRS_ERR_CAPTURE and enqueue
@@ -304,10 +304,10 @@ typedef struct emrs_tuning {
                              device and freed with the plan; when that allocation runs out of
                              memory, the launch searches instead); 0: a binary search bounded by
                              a hint in the kernel arguments */
-  uint32_t warm_tables;   /* with the chunk table, 1 (default): a short kernel reads the chunk table
-                             and the segment descriptors just before each copy, so that the copy's
-                             first load in every workgroup hits the memory-side cache even when the
-                             launch follows unrelated work; 0: the copy alone */
+  uint32_t warm_tables;   /* with the chunk table, 1 (default): the first workgroups of each copy
+                             launch read the chunk table and the segment descriptors, so that the
+                             copy's first load in every workgroup hits the memory-side cache even
+                             when the launch follows unrelated work; 0: the copy alone */
 } emrs_tuning;
 
 int emrs_get_tuning(emrs_tuning *out);
