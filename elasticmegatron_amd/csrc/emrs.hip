@@ -33,6 +33,7 @@
 
 #include "emrs.h"
 #include "internal.h"
+#include "segment.h"
 
 namespace {
 thread_local std::string g_last_error;
@@ -54,7 +55,7 @@ void clear_error() { g_last_error.clear(); }
 
 namespace {
 
-using emrs_internal::fail;
+using namespace emrs_internal;
 
 int hip_fail(hipError_t e, const char *what) {
   return fail(EMRS_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
@@ -130,71 +131,6 @@ struct SegHint {
   uint32_t shift;
 };
 static_assert(2 * sizeof(Bases) + sizeof(SegHint) + 64 <= 4096, "kernel arguments stay under 4 KB");
-
-// Segment as the kernel sees it.  Offsets and strides are in units of
-// (1 << unit_log2) bytes: 16 for the vector path, the element size otherwise.
-// A cast segment (fp32 only) also writes bf16 copies to aux, whose offset and
-// stride are in units of half that size (8 bytes, or one bf16).  A duplicating
-// segment writes its values to aux as well, in the segment's own units.
-struct DevSeg {
-  uint64_t src_off;
-  uint64_t dst_off;
-  uint64_t chunk_begin;  // index of this segment's first chunk
-  uint64_t aux_off;
-  uint32_t len;          // units per row
-  uint32_t rows;
-  uint32_t src_stride;
-  uint32_t dst_stride;
-  uint32_t aux_stride;
-  uint32_t magic;        // row = (t + ((u - t) >> sh1)) >> sh2, t = umulhi(magic, u)
-  // Whole 32-bit words only, so that a workgroup reads its descriptor with
-  // scalar loads alone (the compiler reads 8- and 16-bit fields with vector
-  // loads, which put a vector-memory round trip ahead of the workgroup's data).
-  uint32_t bufs;         // bits 0-15: source buffer; bits 16-31: destination buffer
-  uint32_t meta;         // bits 0-15: second destination (aux) buffer; 16-23: shifts; 24-31: kind
-
-  // shifts: bits 0-4 sh2, bit 5 sh1.  kind: bits 0-2 unit_log2, bits 3-4
-  // elem_log2, bits 5-7 ops.  ops bit 0: also write bf16 to aux; bit 1: write
-  // zeros, read nothing; bit 2: also write the values unchanged to aux.
-  // elem_log2: element size of the input segment (read by the compare kernel
-  // and for duplicates).
-  __host__ __device__ uint32_t src_buf() const { return bufs & 0xffffu; }
-  __host__ __device__ uint32_t dst_buf() const { return bufs >> 16; }
-  __host__ __device__ uint32_t aux_buf() const { return meta & 0xffffu; }
-  __host__ __device__ uint32_t sh1() const { return (meta >> 21) & 1u; }
-  __host__ __device__ uint32_t sh2() const { return (meta >> 16) & 31u; }
-  __host__ __device__ uint32_t unit_log2() const { return (meta >> 24) & 7u; }
-  __host__ __device__ uint32_t elem_log2() const { return (meta >> 27) & 3u; }
-  __host__ __device__ uint32_t ops() const { return meta >> 29; }
-  void set_bufs(uint32_t src, uint32_t dst, uint32_t aux) {
-    bufs = (src & 0xffffu) | (dst << 16);
-    meta = (meta & 0xffff0000u) | (aux & 0xffffu);
-  }
-  void set_kind(uint32_t sh2_, uint32_t sh1_, uint32_t unit_log2_, uint32_t elem_log2_, uint32_t ops_) {
-    meta = (meta & 0xffffu) | ((sh2_ | (sh1_ << 5)) << 16) | ((unit_log2_ | (elem_log2_ << 3) | (ops_ << 5)) << 24);
-  }
-};
-static_assert(sizeof(DevSeg) == 64, "DevSeg layout");
-
-// Division by an invariant divisor (Granlund & Montgomery 1994, fig. 4.1).
-void make_magic(uint32_t d, uint32_t *m, uint32_t *sh1, uint32_t *sh2) {
-  uint32_t l = 0;
-  while ((1ull << l) < d) ++l;
-  uint64_t num = (uint64_t)(((unsigned __int128)1 << 32) * (((unsigned __int128)1 << l) - d) / d) + 1;
-  *m = (uint32_t)num;
-  *sh1 = l < 1 ? l : 1;
-  *sh2 = l > 1 ? l - 1 : 0;
-}
-
-__host__ __device__ __forceinline__ uint32_t umulhi32(uint32_t a, uint32_t b) {
-  return (uint32_t)(((uint64_t)a * b) >> 32);
-}
-
-__host__ __device__ __forceinline__ uint32_t magic_div(uint32_t n, uint32_t m, uint32_t sh1,
-                                                       uint32_t sh2) {
-  uint32_t t = umulhi32(m, n);
-  return (t + ((n - t) >> sh1)) >> sh2;
-}
 
 struct Tuning {
   std::atomic<uint32_t> blocks_per_cu{0};  // persistent grid: 0 = as many as can be resident
@@ -318,6 +254,51 @@ __device__ __forceinline__ void copy_chunk(const DevSeg &s, const char *sbase, c
     }
 }
 
+// Units at any multiple of 2 bytes (the hardware takes them, and the compiler emits whole loads and stores).
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+typedef CastOf<u32x4>::type __attribute__((aligned(2))) u32x2_any;
+
+// Row units [u0, u0 + L * U) of segment s (clipped to u_end) by a workgroup of
+// L lanes, U units per lane, every load issued before the first store.
+template <bool kNT, bool kCast, bool kZero, bool kDup, int L, int U>
+__device__ __forceinline__ void copy_rows(const DevSeg &s, const char *sbase, char *dbase, char *abase, uint32_t u0,
+                                          uint32_t u_end) {
+  const uint32_t lg = s.elem_log2();
+  u32x4 v[U];
+#pragma unroll
+  for (int j = 0; j < U; ++j) {
+    v[j] = u32x4{};
+    if constexpr (!kZero) {
+      const RowUnit r = row_unit(s, dbase, u0 + j * L + threadIdx.x, u_end);
+      if (r.on) v[j] = ld<u32x4_any, kNT>(reinterpret_cast<const u32x4_any *>(sbase + (r.src << lg)));
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < U; ++j) {
+    const RowUnit r = row_unit(s, dbase, u0 + j * L + threadIdx.x, u_end);
+    if (r.on) {
+      st<u32x4_any, kNT>(reinterpret_cast<u32x4_any *>(dbase + (r.dst << lg)), v[j]);
+      if constexpr (kCast)
+        st<u32x2_any, kNT>(reinterpret_cast<u32x2_any *>(abase + (r.aux << 1)), CastOf<u32x4>::cast(v[j]));
+      if constexpr (kDup) st<u32x4_any, kNT>(reinterpret_cast<u32x4_any *>(abase + (r.aux << lg)), v[j]);
+    }
+  }
+}
+
+// copy_rows for what the segment's ops ask for.
+template <bool kNT, int L, int U>
+__device__ __forceinline__ void dispatch_rows(const DevSeg &s, const char *sb, char *db, char *ab, uint32_t u0,
+                                              uint32_t u_end) {
+  switch (s.ops()) {
+    case 0: copy_rows<kNT, false, false, false, L, U>(s, sb, db, ab, u0, u_end); break;
+    case 1: copy_rows<kNT, true, false, false, L, U>(s, sb, db, ab, u0, u_end); break;
+    case 2: copy_rows<kNT, false, true, false, L, U>(s, sb, db, ab, u0, u_end); break;
+    case 3: copy_rows<kNT, true, true, false, L, U>(s, sb, db, ab, u0, u_end); break;
+    case 4: copy_rows<kNT, false, false, true, L, U>(s, sb, db, ab, u0, u_end); break;
+    default: copy_rows<kNT, false, true, true, L, U>(s, sb, db, ab, u0, u_end); break;
+  }
+}
+
 // copy_chunk for the unit width of a segment that carries no bf16 image.
 template <bool kNT, bool kCast, bool kZero, bool kDup>
 __device__ __forceinline__ void dispatch_units(uint32_t ul, const DevSeg &s, const char *sb, char *db, char *ab,
@@ -365,13 +346,17 @@ __device__ __forceinline__ void copy_chunk_run(const DevSeg *__restrict__ segs, 
     }
     // Up to kUnroll chunks of this segment in one step.
     nq = min(min(c_end, s_end) - c, (uint64_t)kUnroll);
-    const uint32_t total = s.len * s.rows;
+    const uint32_t total = s.units();
     const uint32_t u0 = (uint32_t)(c - s.chunk_begin) * kChunkUnits;
     const uint32_t u_end = min(u0 + (uint32_t)nq * kChunkUnits, total);
     const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
     char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
     char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
     const uint32_t ops = s.ops(), ul = s.unit_log2();
+    if (ul == kRowUnits) {
+      dispatch_rows<kNT, kThreads, kUnroll>(s, sb, db, ab, u0, u_end);
+      continue;
+    }
     if (ops & 4) {  // duplicate to aux, with or without zero fill
       if (ops & 2) dispatch_units<kNT, false, true, true>(ul, s, sb, db, ab, u0, u_end);
       else dispatch_units<kNT, false, false, true>(ul, s, sb, db, ab, u0, u_end);
@@ -620,6 +605,8 @@ __device__ __forceinline__ void copy_piece(const DevSeg &s, const char *sb, char
   const uint32_t ops = s.ops(), ul = s.unit_log2();
   if (__builtin_expect(ops == 0 && ul == 4, 1)) {  // most of every plan
     copy_units<u32x4, kNT, false, false, false, L, U>(s, sb, db, ab, u0, total);
+  } else if (ul == kRowUnits) {
+    dispatch_rows<kNT, L, U>(s, sb, db, ab, u0, total);
   } else if (ops & 4) {  // duplicate to aux, with or without zero fill
     if (ops & 2) dispatch_chunk<kNT, true, true, L, U>(ul, s, sb, db, ab, u0, total);
     else dispatch_chunk<kNT, false, true, L, U>(ul, s, sb, db, ab, u0, total);
@@ -638,12 +625,14 @@ __device__ __forceinline__ void copy_piece(const DevSeg &s, const char *sb, char
   }
 }
 
-// copy_piece with every unit width through buffer instructions.
+// copy_piece with every unit width but row units through buffer instructions.
 template <bool kNT, int L, int U>
 __device__ __forceinline__ void copy_piece_buf(const DevSeg &s, const char *sb, char *db, char *ab, uint32_t u0,
                                                uint32_t total) {
   const uint32_t ops = s.ops(), ul = s.unit_log2();
-  if (ops & 4) {
+  if (ul == kRowUnits) {
+    dispatch_rows<kNT, L, U>(s, sb, db, ab, u0, total);
+  } else if (ops & 4) {
     if (ops & 2) dispatch_chunk_buf<kNT, true, true, L, U>(ul, s, sb, db, ab, u0, total);
     else dispatch_chunk_buf<kNT, false, true, L, U>(ul, s, sb, db, ab, u0, total);
   } else if (ops & 1) {  // with the bf16 image (fp32 only: 16- or 4-byte units)
@@ -754,7 +743,7 @@ __global__ __launch_bounds__(L) void copy_plan_kernel(const DevSeg *__restrict__
     }
   }
   const DevSeg s = segs[lo];
-  const uint32_t total = s.len * s.rows;
+  const uint32_t total = s.units();
   const uint32_t u0 = (uint32_t)(c - s.chunk_begin) * kChunkUnits + (uint32_t)(w % kPieces) * (L * U);
   if (kPieces > 1 && u0 >= total) return;
   const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
@@ -794,7 +783,7 @@ __global__ __launch_bounds__(L) void copy_pieces_kernel(const uint32_t *__restri
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;
   const DevSeg s = load_seg(segs + chunk_seg[c]);
-  const uint32_t total = s.len * s.rows;
+  const uint32_t total = s.units();
   const uint32_t u0 = (uint32_t)(c - s.chunk_begin) * kChunkUnits + (uint32_t)(w % kPieces) * (L * U);
   const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
   char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
@@ -998,20 +987,20 @@ struct Builder {
   uint64_t chunks = 0;
   uint64_t vec_bytes = 0, scalar_bytes = 0;
 
-  // A copy in units of (1 << ul) bytes, optionally with its bf16 image.
-  // Splits to the kernel's 32-bit limits.
+  // A copy whose offsets, length and strides count (1 << ul) bytes, optionally
+  // with its bf16 image; `by_rows`: in row units.  Splits to the kernel's
+  // 32-bit limits.
   void emit(uint32_t sbuf, uint32_t dbuf, uint32_t ul, uint64_t so, uint64_t dof, uint64_t len,
-            uint64_t rows, uint64_t ss, uint64_t ds, Aux ax = Aux()) {
+            uint64_t rows, uint64_t ss, uint64_t ds, Aux ax = Aux(), bool by_rows = false) {
     if (len == 0 || rows == 0) return;
     if (rows > 1 && ss == len && ds == len && (!ax.on || ax.stride == len)) {  // contiguous
       len *= rows;
       rows = 1;
     }
-    (ul == 4 ? vec_bytes : scalar_bytes) += (len * rows) << ul;
     if (rows == 1) {
       for (uint64_t off = 0; off < len; off += kMaxUnitsPerSeg) {
         const uint64_t n = std::min<uint64_t>(kMaxUnitsPerSeg, len - off);
-        push(sbuf, dbuf, ul, so + off, dof + off, (uint32_t)n, 1, 0, 0, ax, ax.off + off, 0);
+        push(sbuf, dbuf, ul, so + off, dof + off, (uint32_t)n, 1, 0, 0, ax, ax.off + off, 0, by_rows);
       }
       return;
     }
@@ -1023,7 +1012,7 @@ struct Builder {
         for (uint64_t off = 0; off < len; off += kMaxUnitsPerSeg) {
           const uint64_t n = std::min<uint64_t>(kMaxUnitsPerSeg, len - off);
           push(sbuf, dbuf, ul, so + r * ss + off, dof + r * ds + off, (uint32_t)n, 1, 0, 0, ax,
-               ax.off + r * ax.stride + off, 0);
+               ax.off + r * ax.stride + off, 0, by_rows);
         }
       return;
     }
@@ -1031,12 +1020,12 @@ struct Builder {
     for (uint64_t r = 0; r < rows; r += rows_per) {
       const uint64_t n = std::min<uint64_t>(rows_per, rows - r);
       push(sbuf, dbuf, ul, so + r * ss, dof + r * ds, (uint32_t)len, (uint32_t)n, (uint32_t)ss, (uint32_t)ds,
-           ax, ax.off + r * ax.stride, (uint32_t)ax.stride);
+           ax, ax.off + r * ax.stride, (uint32_t)ax.stride, by_rows);
     }
   }
 
   void push(uint32_t sbuf, uint32_t dbuf, uint32_t ul, uint64_t so, uint64_t dof, uint32_t len, uint32_t rows,
-            uint32_t ss, uint32_t ds, const Aux &ax, uint64_t aoff, uint32_t astride) {
+            uint32_t ss, uint32_t ds, const Aux &ax, uint64_t aoff, uint32_t astride, bool by_rows) {
     DevSeg d{};
     d.src_off = so;
     d.dst_off = dof;
@@ -1045,15 +1034,18 @@ struct Builder {
     d.rows = rows;
     d.src_stride = rows > 1 ? ss : 0;
     d.dst_stride = rows > 1 ? ds : 0;
-    uint32_t sh1 = 0, sh2 = 0;
-    make_magic(len, &d.magic, &sh1, &sh2);
     const uint32_t ops = (ax.cast ? 1u : 0u) | (ax.zero ? 2u : 0u) | (ax.dup ? 4u : 0u);
-    d.set_kind(sh2, sh1, ul, cur_elem_log2, ops);
+    const uint64_t row_bytes = (uint64_t)len << ul;
+    // A last piece under 16 bytes of a row cut at kMaxUnitsPerSeg goes element by element.
+    const bool row_units = by_rows && row_bytes >= 16;
+    d.set_kind(row_units ? kRowUnits : ul, cur_elem_log2, ops, row_units && row_bytes >= kLineRowBytes);
+    uint32_t magic = 0, sh1 = 0, sh2 = 0;
+    make_magic(d.row_units(), &magic, &sh1, &sh2);
+    d.set_division(magic, sh1, sh2);
     d.set_bufs(sbuf, dbuf, ax.on ? ax.buf : dbuf);
     d.aux_off = ax.on ? aoff : 0;
     d.aux_stride = ax.on && rows > 1 ? astride : 0;
-    const uint64_t units = (uint64_t)len * rows;
-    chunks += (units + kChunkUnits - 1) / kChunkUnits;
+    chunks += ((uint64_t)d.units() + kChunkUnits - 1) / kChunkUnits;
     out.push_back(d);
     origin.push_back(cur_origin);
   }
@@ -1274,7 +1266,7 @@ int resolved_table(emrs_plan *plan, int dev, const ResolvedBases &rb, hipStream_
     auto units_from_lo = [lo](uint64_t p, uint32_t log2) -> uint64_t { return p >= lo ? (p - lo) >> log2 : 0; };
     std::vector<DevSeg> segs = plan->segs;
     for (DevSeg &d : segs) {
-      const uint32_t ul = d.unit_log2(), ops = d.ops();
+      const uint32_t ul = d.off_log2(), ops = d.ops();
       const uint32_t aux_log2 = (ops & 1) ? ul - 1 : ul;  // a bf16 image unit is half a unit
       d.src_off = (ops & 2) ? 0 : d.src_off + units_from_lo(rb.ptrs[d.src_buf()], ul);
       d.dst_off += units_from_lo(rb.ptrs[ns + d.dst_buf()], ul);
@@ -1397,15 +1389,17 @@ __device__ __forceinline__ void cmp_float(LaneAcc &a, uint32_t e_bits, uint32_t 
   a.max_rel = fmaxf(a.max_rel, d / (fabsf(e) + 1e-12f));
 }
 
-// Compare one unit (1, 2, 4, 8 or 16 bytes held in w[0..3]) element by element.
+// Compare one unit (1, 2, 4, 8 or 16 bytes held in w[0..3]) element by element: its elements [first, last).
 __device__ __forceinline__ void cmp_words(LaneAcc &a, const uint32_t *e, const uint32_t *g, uint32_t unit_bytes,
-                                          uint32_t elem_log2) {
+                                          uint32_t elem_log2, uint32_t first = 0, uint32_t last = 16) {
   switch (elem_log2) {
     case 2:  // fp32
-      for (uint32_t k = 0; k < unit_bytes / 4; ++k) cmp_float(a, e[k], g[k]);
+      for (uint32_t k = 0; k < unit_bytes / 4; ++k)
+        if (k >= first && k < last) cmp_float(a, e[k], g[k]);
       break;
     case 1:  // bf16
       for (uint32_t k = 0; k < unit_bytes / 2; ++k) {
+        if (k < first || k >= last) continue;
         const uint32_t sh = (k & 1) * 16;
         cmp_float(a, ((e[k >> 1] >> sh) & 0xffffu) << 16, ((g[k >> 1] >> sh) & 0xffffu) << 16);
       }
@@ -1418,7 +1412,7 @@ __device__ __forceinline__ void cmp_words(LaneAcc &a, const uint32_t *e, const u
       break;
     default:  // 8-byte elements: bits only
       for (uint32_t k = 0; k < unit_bytes / 8; ++k)
-        a.mismatches += (e[2 * k] != g[2 * k]) || (e[2 * k + 1] != g[2 * k + 1]);
+        if (k >= first && k < last) a.mismatches += (e[2 * k] != g[2 * k]) || (e[2 * k + 1] != g[2 * k + 1]);
       break;
   }
 }
@@ -1483,6 +1477,35 @@ __device__ __forceinline__ void compare_chunk(const DevSeg &s, const char *sbase
         aux_words_of(ld<A, true>(aux + ao), ga);
         cmp_words(x, ea, ga, (uint32_t)sizeof(A), 1);
       }
+    }
+  }
+}
+
+// compare_chunk for row units: every element of a row once, whichever units hold it.
+__device__ __forceinline__ void compare_rows(const DevSeg &s, const char *sbase, const char *dbase, const char *abase,
+                                             uint32_t u0, uint32_t u_end, LaneAcc &m, LaneAcc &x) {
+  const uint32_t ops = s.ops(), lg = s.elem_log2();
+  for (uint32_t j = 0; j < kUnroll; ++j) {
+    const RowUnit r = row_unit(s, dbase, u0 + j * kThreads + threadIdx.x, u_end);
+    if (!r.on) continue;
+    u32x4 e = u32x4{};
+    if (!(ops & 2)) e = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(sbase + (r.src << lg)));
+    const u32x4 g = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(dbase + (r.dst << lg)));
+    uint32_t ew[4], gw[4];
+    words_of(e, ew);
+    words_of(g, gw);
+    cmp_words(m, ew, gw, 16, lg, r.first, r.last);
+    if (ops & 4) {
+      const u32x4 d = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(abase + (r.aux << lg)));
+      words_of(d, gw);
+      cmp_words(x, ew, gw, 16, lg, r.first, r.last);
+    }
+    if (ops & 1) {
+      const CastOf<u32x4>::type a = ld<u32x2_any, true>(reinterpret_cast<const u32x2_any *>(abase + (r.aux << 1)));
+      uint32_t ea[2], ga[2];
+      aux_words_of(CastOf<u32x4>::cast(e), ea);
+      aux_words_of(a, ga);
+      cmp_words(x, ea, ga, 8, 1, r.first, r.last);
     }
   }
 }
@@ -1588,6 +1611,38 @@ __device__ __forceinline__ void differ_units(const DevSeg &s, const char *sbase,
   }
 }
 
+// The bit-level pass over row units [u0, u0 + L * U) (clipped to u_end), every
+// load issued before the comparison.  Elements that two units hold are looked at twice.
+template <int L, int U>
+__device__ __forceinline__ void differ_rows(const DevSeg &s, const char *sbase, const char *dbase, const char *abase,
+                                            uint32_t u0, uint32_t u_end, uint32_t &dm, uint32_t &dx) {
+  const uint32_t ops = s.ops(), lg = s.elem_log2();
+  u32x4 e[U], g[U];
+#pragma unroll
+  for (int j = 0; j < U; ++j) {
+    const RowUnit r = row_unit(s, dbase, u0 + j * L + threadIdx.x, u_end);
+    e[j] = g[j] = u32x4{};
+    if (r.on) {
+      if (!(ops & 2)) e[j] = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(sbase + (r.src << lg)));
+      g[j] = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(dbase + (r.dst << lg)));
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < U; ++j) {
+    dm |= differ(e[j], g[j]);
+    if (!(ops & 5)) continue;
+    const RowUnit r = row_unit(s, dbase, u0 + j * L + threadIdx.x, u_end);
+    if (!r.on) continue;
+    if (ops & 4) {
+      const u32x4 d = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(abase + (r.aux << lg)));
+      dx |= differ(e[j], d);
+    } else {
+      const CastOf<u32x4>::type a = ld<u32x2_any, true>(reinterpret_cast<const u32x2_any *>(abase + (r.aux << 1)));
+      dx |= differ(CastOf<u32x4>::cast(e[j]), a);
+    }
+  }
+}
+
 template <bool kTable, int U>
 __global__ __launch_bounds__(64) void differ_piece_kernel(
     const DevSeg *__restrict__ segs, uint64_t n_chunks, Bases src, Bases dst, const uint64_t *__restrict__ src_tab,
@@ -1600,7 +1655,7 @@ __global__ __launch_bounds__(64) void differ_piece_kernel(
   if (c >= n_chunks) return;
   const uint32_t lo = chunk_seg[c];
   const DevSeg s = segs[lo];
-  const uint32_t total = s.len * s.rows;
+  const uint32_t total = s.units();
   const uint32_t u0 = (uint32_t)(c - s.chunk_begin) * kChunkUnits + (uint32_t)(w % kPieces) * (64 * U);
   if (kPieces > 1 && u0 >= total) return;
   const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
@@ -1608,6 +1663,7 @@ __global__ __launch_bounds__(64) void differ_piece_kernel(
   const char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
   uint32_t dm = 0, dx = 0;
   switch (s.unit_log2()) {
+    case kRowUnits: differ_rows<64, U>(s, sb, db, ab, u0, total, dm, dx); break;
     case 4: differ_units<u32x4, U>(s, sb, db, ab, u0, total, dm, dx); break;
     case 3: differ_units<uint64_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
     case 2: differ_units<uint32_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
@@ -1670,13 +1726,14 @@ __global__ __launch_bounds__(kThreads) void differ_plan_kernel(
       cur_g = g;
       cur_ga = ga;
       cur_aux = aux;
-      const uint32_t total = s.len * s.rows;
+      const uint32_t total = s.units();
       const uint32_t u0 = (uint32_t)(q - s.chunk_begin) * kChunkUnits;
       const uint32_t u_end = min(u0 + (uint32_t)nq * kChunkUnits, total);
       const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
       const char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
       const char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
       switch (s.unit_log2()) {
+        case kRowUnits: differ_rows<kThreads, kUnroll>(s, sb, db, ab, u0, u_end, dm, dx); break;
         case 4: differ_chunk<u32x4>(s, sb, db, ab, u0, u_end, dm, dx); break;
         case 3: differ_chunk<uint64_t>(s, sb, db, ab, u0, u_end, dm, dx); break;
         case 2: differ_chunk<uint32_t>(s, sb, db, ab, u0, u_end, dm, dx); break;
@@ -1797,13 +1854,14 @@ __global__ __launch_bounds__(kThreads) void compare_plan_kernel(
       cur_g = g;
       cur_ga = ga;
       cur_aux = aux;
-      const uint32_t total = s.len * s.rows;
+      const uint32_t total = s.units();
       const uint32_t u0 = (uint32_t)(q - s.chunk_begin) * kChunkUnits;
       const uint32_t u_end = min(u0 + (uint32_t)nq * kChunkUnits, total);
       const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
       const char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
       const char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
       switch (s.unit_log2()) {
+        case kRowUnits: compare_rows(s, sb, db, ab, u0, u_end, m, x); break;
         case 4: compare_chunk<u32x4>(s, sb, db, ab, u0, u_end, m, x); break;
         case 3: compare_chunk<uint64_t>(s, sb, db, ab, u0, u_end, m, x); break;
         case 2: compare_chunk<uint32_t>(s, sb, db, ab, u0, u_end, m, x); break;
@@ -1853,10 +1911,9 @@ int compare_setup(emrs_plan *plan, void *const *src_bases, void *const *dst_base
     const uint32_t g = groups ? groups[o] : 0, ga = aux_groups ? aux_groups[o] : g;
     job->g_host[k] = g;
     job->g_host[nd + k] = ga;
-    const uint64_t units = (uint64_t)d.len * d.rows;
-    elements[g] += units << (d.unit_log2() - d.elem_log2());
-    if (d.ops() & 1) elements[ga] += units << (d.unit_log2() - 2);
-    if (d.ops() & 4) elements[ga] += units << (d.unit_log2() - d.elem_log2());
+    const uint64_t n = ((uint64_t)d.len * d.rows) << (d.off_log2() - d.elem_log2());
+    elements[g] += n;
+    if (d.ops() & 5) elements[ga] += n;
   }
   for (uint32_t g = 0; g < n_groups; ++g) {
     stats[g] = emrs_compare_stats{};
@@ -2098,35 +2155,38 @@ int emrs_plan_create(const emrs_segment *segs, uint64_t n_segs, const uint64_t *
     const uint64_t avu = has_aux ? 16 * aeb / eb : 16;
     const bool aux_vec_ok = !has_aux || (ao % avu == 0 && as % avu == 0);
     const bool rows1 = s.rows == 1 || (ss == lb && ds == lb && (!has_aux || as == s.len * aeb));
-    if (rows1) {
-      const uint64_t L = lb * s.rows;  // contiguous bytes
-      if (so % 16 == 0 && dof % 16 == 0 && L % 16 == 0 && aux_vec_ok) {
-        ax.off = ao / avu;
-        bld.emit(s.src_buf, s.dst_buf, 4, so / 16, dof / 16, L / 16, 1, 0, 0, ax);
-      } else if (so % 16 == dof % 16 && (!has_aux || (ao % avu) * eb / aeb == so % 16)) {
-        // Source, destination and aux reach a 16-byte boundary at the same element.
-        const uint64_t head = std::min<uint64_t>((16 - so % 16) % 16, L);
-        const uint64_t body = (L - head) / 16 * 16;
-        const uint64_t tail = L - head - body;
-        const uint64_t aux_head = head * aeb / eb, aux_body = body * aeb / eb;
-        ax.off = has_aux ? ao / aeb : 0;
-        bld.emit(s.src_buf, s.dst_buf, lg, so / eb, dof / eb, head / eb, 1, 0, 0, ax);
-        ax.off = has_aux ? (ao + aux_head) / avu : 0;
-        bld.emit(s.src_buf, s.dst_buf, 4, (so + head) / 16, (dof + head) / 16, body / 16, 1, 0, 0, ax);
-        ax.off = has_aux ? (ao + aux_head + aux_body) / aeb : 0;
-        bld.emit(s.src_buf, s.dst_buf, lg, (so + head + body) / eb, (dof + head + body) / eb, tail / eb, 1, 0, 0, ax);
-      } else {
-        ax.off = s.aux_off;
-        bld.emit(s.src_buf, s.dst_buf, lg, so / eb, s.dst_off, L / eb, 1, 0, 0, ax);
-      }
-    } else if (so % 16 == 0 && dof % 16 == 0 && lb % 16 == 0 && ss % 16 == 0 && ds % 16 == 0 && aux_vec_ok) {
-      ax.off = ao / avu;
-      ax.stride = as / avu;
-      bld.emit(s.src_buf, s.dst_buf, 4, so / 16, dof / 16, lb / 16, s.rows, ss / 16, ds / 16, ax);
+    const uint64_t L = lb * s.rows;
+    // One run of L bytes, or rows of lb bytes.
+    const uint64_t run = rows1 ? L : lb;
+    const bool all16 = so % 16 == 0 && dof % 16 == 0 && run % 16 == 0 && (rows1 || (ss % 16 == 0 && ds % 16 == 0)) &&
+                       aux_vec_ok;
+    // Source, destination and aux reach a 16-byte boundary at the same element.
+    const bool together = rows1 && so % 16 == dof % 16 && (!has_aux || (ao % avu) * eb / aeb == so % 16);
+    const uint64_t head = std::min<uint64_t>((16 - so % 16) % 16, run);
+    bld.vec_bytes += all16 ? L : (together ? (L - head) / 16 * 16 : 0);
+    bld.scalar_bytes += all16 ? 0 : (together ? L - (L - head) / 16 * 16 : L);
+    // Row units (see kRowUnits) wherever 16-byte units do not fit.  Where they
+    // do fit they stay, on lines or not: row units gained 0-1% on segments off
+    // the lines of large plans, but cost 8% on the tiny model's TP2 -> TP1 switch
+    // and 7% on a 1.9 GB one.  Byte elements stay on the element path: no tensor
+    // of a training state has them.
+    const bool by_rows = lg > 0 && !all16 && run >= 16;
+    const uint32_t ul = by_rows ? (uint32_t)lg : (all16 ? 4u : (uint32_t)lg);
+    const uint64_t ub = 1ull << ul, aub = has_aux ? ub * aeb / eb : 1;  // bytes per unit, and per aux unit
+    if (has_aux) ax.off = ao / aub;
+    if (rows1 && !by_rows && !all16 && together) {  // byte elements: a vector body between two ends
+      const uint64_t body = (L - head) / 16 * 16, tail = L - head - body;
+      const uint64_t aux_head = head * aeb / eb, aux_body = body * aeb / eb;
+      bld.emit(s.src_buf, s.dst_buf, lg, so / eb, dof / eb, head / eb, 1, 0, 0, ax);
+      ax.off = has_aux ? (ao + aux_head) / avu : 0;
+      bld.emit(s.src_buf, s.dst_buf, 4, (so + head) / 16, (dof + head) / 16, body / 16, 1, 0, 0, ax);
+      ax.off = has_aux ? (ao + aux_head + aux_body) / aeb : 0;
+      bld.emit(s.src_buf, s.dst_buf, lg, (so + head + body) / eb, (dof + head + body) / eb, tail / eb, 1, 0, 0, ax);
+    } else if (rows1) {
+      bld.emit(s.src_buf, s.dst_buf, ul, so / ub, dof / ub, L / ub, 1, 0, 0, ax, by_rows);
     } else {
-      ax.off = s.aux_off;
-      ax.stride = s.rows > 1 ? s.aux_stride : 0;
-      bld.emit(s.src_buf, s.dst_buf, lg, so / eb, s.dst_off, s.len, s.rows, ss / eb, s.dst_stride, ax);
+      ax.stride = has_aux ? as / aub : 0;
+      bld.emit(s.src_buf, s.dst_buf, ul, so / ub, dof / ub, lb / ub, s.rows, ss / ub, ds / ub, ax, by_rows);
     }
   }
   if (flags & EMRS_PLAN_CHECK_DISJOINT) {

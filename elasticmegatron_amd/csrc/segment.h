@@ -1,0 +1,152 @@
+// Device segments: the descriptors a copy plan is lowered to, and the arithmetic
+// that places a lane's unit in them.  Plain C++ as well, so that it can be
+// checked on the host.
+#ifndef EMRS_SEGMENT_H
+#define EMRS_SEGMENT_H
+
+#include <cstdint>
+
+#ifdef __HIPCC__
+#include <hip/hip_runtime.h>
+#define EMRS_HD __host__ __device__
+#else
+#define EMRS_HD
+#endif
+
+namespace emrs_internal {
+
+// A segment's unit: 2^unit_log2 bytes, one per lane, at multiples of its size
+// (16 bytes: the vector path; an element: the element path); or kRowUnits:
+// 16 bytes anywhere in a row, for rows of at least 16 bytes whose source,
+// destination or length is no whole number of 16-byte units.  Row units follow
+// the destination: unit k of a row holds the row's bytes
+// [16k - p, 16k - p + 16), p being the row's distance from the 128-byte line
+// (or, in rows under kLineRowBytes, from the 16-byte boundary) before it, so
+// whole lines are written by one workgroup each and inner stores are aligned;
+// the loads are not, and read a line twice where a workgroup ends inside it.
+// A unit that reaches over an end of the row is moved inside it: it then writes
+// again, with the same values, bytes that the next or previous unit writes.
+// Every row has units for the largest possible p; those past its end idle.
+// The element path that these segments took before moves 64 elements per
+// workgroup and is bound by launching them.  Measured, before and now (12 GiB
+// copied, one process): fp32 one element off 2.36 and 6.49 TB/s; bf16 one
+// element off 1.22 and 6.23; rows of 667 fp32 gathered 2.41 and 6.20,
+// scattered 2.39 and 5.77, gathered with their bf16 image 2.88 and 5.63.  A
+// 24-layer model of hidden size 1000, TP1 DP8 -> TP4 DP2 (9.2 GB): 1805 us
+// and 1494 us.
+constexpr uint32_t kRowUnits = 5;
+constexpr uint64_t kLineRowBytes = 512;
+
+// Segment as the kernel sees it.  Offsets and strides are in units of
+// (1 << unit_log2) bytes: 16 for the vector path, the element size otherwise
+// (row units too, whose len also counts elements).
+// A cast segment (fp32 only) also writes bf16 copies to aux, whose offset and
+// stride are in units of half that size (8 bytes, or one bf16).  A duplicating
+// segment writes its values to aux as well, in the segment's own units.
+struct DevSeg {
+  uint64_t src_off;
+  uint64_t dst_off;
+  uint64_t chunk_begin;  // index of this segment's first chunk
+  uint64_t aux_off;
+  uint32_t len;          // units per row
+  uint32_t rows;
+  uint32_t src_stride;
+  uint32_t dst_stride;
+  uint32_t aux_stride;
+  uint32_t magic;        // row = (t + ((u - t) >> sh1)) >> sh2, t = umulhi(magic, u)
+  // Whole 32-bit words only, so that a workgroup reads its descriptor with
+  // scalar loads alone (the compiler reads 8- and 16-bit fields with vector
+  // loads, which put a vector-memory round trip ahead of the workgroup's data).
+  uint32_t bufs;         // bits 0-15: source buffer; bits 16-31: destination buffer
+  uint32_t meta;         // bits 0-15: second destination (aux) buffer; 16-23: shifts; 24-31: kind
+
+  // shifts: bits 0-4 sh2, bit 5 sh1, bit 6 row units on lines (else on 16-byte
+  // boundaries).  kind: bits 0-2 unit_log2 (or kRowUnits), bits 3-4
+  // elem_log2, bits 5-7 ops.  ops bit 0: also write bf16 to aux; bit 1: write
+  // zeros, read nothing; bit 2: also write the values unchanged to aux.
+  // elem_log2: element size of the input segment (read by the compare kernel
+  // and for duplicates).
+  EMRS_HD uint32_t src_buf() const { return bufs & 0xffffu; }
+  EMRS_HD uint32_t dst_buf() const { return bufs >> 16; }
+  EMRS_HD uint32_t aux_buf() const { return meta & 0xffffu; }
+  EMRS_HD uint32_t sh1() const { return (meta >> 21) & 1u; }
+  EMRS_HD uint32_t sh2() const { return (meta >> 16) & 31u; }
+  EMRS_HD uint32_t unit_log2() const { return (meta >> 24) & 7u; }
+  EMRS_HD uint32_t elem_log2() const { return (meta >> 27) & 3u; }
+  EMRS_HD uint32_t ops() const { return meta >> 29; }
+  void set_bufs(uint32_t src, uint32_t dst, uint32_t aux) {
+    bufs = (src & 0xffffu) | (dst << 16);
+    meta = (meta & 0xffff0000u) | (aux & 0xffffu);
+  }
+  // Bytes a row unit's phase is counted from, less one.
+  EMRS_HD uint32_t phase_mask() const { return (meta >> 22) & 1u ? 127u : 15u; }
+  // Units in a row, and in the segment.
+  EMRS_HD uint32_t row_units() const {
+    if (unit_log2() != kRowUnits) return len;
+    const uint32_t lg = elem_log2();
+    return (len + (phase_mask() >> lg) + (15u >> lg)) >> (4 - lg);
+  }
+  EMRS_HD uint32_t units() const { return row_units() * rows; }
+  // log2 of the bytes that offsets and strides count.
+  EMRS_HD uint32_t off_log2() const { return unit_log2() == kRowUnits ? elem_log2() : unit_log2(); }
+  void set_kind(uint32_t unit_log2_, uint32_t elem_log2_, uint32_t ops_, bool on_lines) {
+    meta = (meta & 0x003fffffu) | ((on_lines ? 1u : 0u) << 22) |
+           ((unit_log2_ | (elem_log2_ << 3) | (ops_ << 5)) << 24);
+  }
+  void set_division(uint32_t magic_, uint32_t sh1_, uint32_t sh2_) {
+    magic = magic_;
+    meta = (meta & ~(63u << 16)) | ((sh2_ | (sh1_ << 5)) << 16);
+  }
+};
+static_assert(sizeof(DevSeg) == 64, "DevSeg layout");
+
+// Division by an invariant divisor (Granlund & Montgomery 1994, fig. 4.1).
+inline void make_magic(uint32_t d, uint32_t *m, uint32_t *sh1, uint32_t *sh2) {
+  uint32_t l = 0;
+  while ((1ull << l) < d) ++l;
+  uint64_t num = (uint64_t)(((unsigned __int128)1 << 32) * (((unsigned __int128)1 << l) - d) / d) + 1;
+  *m = (uint32_t)num;
+  *sh1 = l < 1 ? l : 1;
+  *sh2 = l > 1 ? l - 1 : 0;
+}
+
+EMRS_HD inline uint32_t umulhi32(uint32_t a, uint32_t b) {
+  return (uint32_t)(((uint64_t)a * b) >> 32);
+}
+
+EMRS_HD inline uint32_t magic_div(uint32_t n, uint32_t m, uint32_t sh1,
+                                                       uint32_t sh2) {
+  uint32_t t = umulhi32(m, n);
+  return (t + ((n - t) >> sh1)) >> sh2;
+}
+
+// Where row unit `u` of segment `s` lies: element offsets from the bases, and
+// the elements [first, last) of the unit that no other unit holds as well.
+// on = false: an idle unit.
+struct RowUnit {
+  uint64_t src, dst, aux;
+  uint32_t first, last;
+  bool on;
+};
+EMRS_HD inline RowUnit row_unit(const DevSeg &s, const char *dbase, uint32_t u, uint32_t u_end) {
+  const uint32_t lg = s.elem_log2(), per = 16u >> lg, upr = s.row_units();
+  uint32_t row = 0;
+  if (s.rows > 1) row = magic_div(u, s.magic, s.sh1(), s.sh2());
+  RowUnit r;
+  r.dst = s.dst_off + (uint64_t)row * s.dst_stride;
+  const uint32_t p = ((uint32_t)(uintptr_t)dbase + ((uint32_t)r.dst << lg)) & s.phase_mask();
+  const int32_t at = (int32_t)((u - row * upr) * per) - (int32_t)(p >> lg), len = (int32_t)s.len;
+  const int32_t end = len - (int32_t)per;  // last place of a unit
+  const int32_t col = at < 0 ? 0 : (at < end ? at : end);
+  r.on = u < u_end && at > -(int32_t)per && at < len;
+  r.first = (uint32_t)((at < 0 ? 0 : at) - col);
+  r.last = (uint32_t)((at + (int32_t)per < len ? at + (int32_t)per : len) - col);
+  r.src = s.src_off + (uint64_t)row * s.src_stride + col;
+  r.dst += col;
+  r.aux = s.aux_off + (uint64_t)row * s.aux_stride + col;
+  return r;
+}
+
+}  // namespace emrs_internal
+
+#endif  // EMRS_SEGMENT_H

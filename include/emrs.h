@@ -117,8 +117,10 @@ typedef struct emrs_plan_stats {
   uint64_t n_device_segments; /* after alignment splitting */
   uint64_t payload_bytes;   /* bytes written per execution, bf16 images and duplicates included */
   uint64_t read_bytes;      /* bytes read per execution */
-  uint64_t vector_bytes;    /* bytes written through 16-byte units (second destinations excluded) */
-  uint64_t scalar_bytes;    /* bytes written element by element (second destinations excluded) */
+  uint64_t vector_bytes;    /* bytes whose source and destination fill 16-byte units together (second
+                               destinations excluded) */
+  uint64_t scalar_bytes;    /* the other bytes: moved in 16-byte units that follow the destination where
+                               a row holds 16 bytes and its elements 2 or more, else element by element */
   uint64_t n_chunks;        /* work chunks per execution */
   uint32_t n_src_bufs;
   uint32_t n_dst_bufs;
@@ -295,9 +297,9 @@ typedef struct emrs_tuning {
   uint32_t units;         /* 16-byte units per lane, 1 (default), 2 or 4, with lanes * units
                              dividing 256: a chunk of 256 units is split into 256 / (lanes * units)
                              pieces, one workgroup each (0: 256 / lanes, one workgroup per chunk) */
-  uint32_t buffer_ops;    /* one workgroup per piece, 1: 16-byte units are moved with buffer
-                             instructions (32-bit offsets from a per-piece base); 0: with 64-bit
-                             global addresses */
+  uint32_t buffer_ops;    /* one workgroup per piece, 1: units at multiples of their size are moved
+                             with buffer instructions (32-bit offsets from a per-piece base); 0: with
+                             64-bit global addresses */
   uint32_t chunk_index;   /* one workgroup per piece, 1 (default): each workgroup reads its
                              segment from the plan's chunk table (4 * emrs_plan_stats.n_chunks
                              bytes of device memory, made on the plan's first such call on a
