@@ -693,9 +693,9 @@ __device__ __forceinline__ void warm_tables(const uint32_t *chunk_seg, const Dev
 // schedule: L = 64, U = 1, four 1 KB pieces per chunk).  A chunk of 256 units
 // holds 256 / (L * U) pieces; workgroup w takes piece w % that of chunk
 // w / that, and a piece past the end of its segment's last chunk does
-// nothing.  The grid is two-dimensional (w = blockIdx.y * gridDim.x +
-// blockIdx.x) because one dimension holds fewer than 2^32 lanes; workgroups
-// past the last piece exit at once.  The segment depends on the chunk alone,
+// nothing.  Past the 2^32 - 1 lanes of one dimension the grid has rows
+// (w = blockIdx.y * gridDim.x + blockIdx.x); workgroups past the last piece
+// exit at once.  The segment depends on the chunk alone,
 // so finding it runs on the scalar unit, once per wave: one load from the
 // plan's chunk table (chunk_seg, by default), or a binary search whose upper
 // levels stay in the scalar cache for every workgroup in flight.  With the
@@ -1879,6 +1879,22 @@ __global__ void clear_words_kernel(uint32_t *p, uint64_t n) {
     p[i] = 0;
 }
 
+// A grid of `n_wg` workgroups of `lanes` lanes, with fewer than 8 more per row:
+// one row up to the 2^32 - 1 lanes that a dimension holds, else as many equal
+// rows as that takes, each a multiple of 8 workgroups long so that a
+// workgroup's XCD follows from its number.  Rows of 65536 workgroups were used
+// before: the last one, half empty on average, still cost its launch, 0.4 ns a
+// workgroup (a 383 MB switch 65.9 us, of which 14 us for the 36,000 empty
+// workgroups of its last row).  False when 65535 rows do not hold them.
+bool tight_grid(uint64_t n_wg, uint32_t lanes, dim3 *grid) {
+  const uint64_t max_x = 0xffffffffull / lanes / 8 * 8;
+  const uint64_t rows = std::max<uint64_t>(1, (n_wg + max_x - 1) / max_x);
+  if (rows > kMaxGridY) return false;
+  const uint64_t gx = rows == 1 ? n_wg : std::min(max_x, ((n_wg + rows - 1) / rows + 7) / 8 * 8);
+  *grid = dim3((uint32_t)gx, (uint32_t)((n_wg + gx - 1) / gx));
+  return true;
+}
+
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // What both comparison entry points prepare on the host: checked bases, the
@@ -1962,8 +1978,8 @@ hipError_t compare_launch(const emrs_plan *plan, const CompareJob &job, const De
   if (!active && job.cseg) {  // the first pass on the copy kernel's schedule
     constexpr int U = 4;
     const uint64_t n_wg = plan->n_chunks * (kChunkUnits / (64 * U));
-    const uint64_t gx = std::min<uint64_t>(n_wg, std::max<uint64_t>(1ull << 16, (n_wg + kMaxGridY - 1) / kMaxGridY));
-    const dim3 pgrid((uint32_t)gx, (uint32_t)((n_wg + gx - 1) / gx));
+    dim3 pgrid;
+    if (!tight_grid(n_wg, 64, &pgrid)) return hipErrorInvalidConfiguration;
     const uint32_t remap = g_tuning.xcd_remap.load();
     const bool by_xcd = remap == 2 || (remap == 1 && plan->n_chunks >= kXcdRemapMinChunks);
     const uint64_t xcd_share = by_xcd ? n_wg / 8 : 0;
@@ -2267,12 +2283,9 @@ int launch_chunks(const CopyLaunch &c) {
     n_warm = ((units + kWarmUnits * L - 1) / (kWarmUnits * L) + 7) / 8 * 8;
     if (n_warm > 0xffffffffull) n_warm = 0;
   }
-  // A grid of at most 65535 rows, each a multiple of 8 workgroups long when there are several.
-  const uint64_t n_wg = n_warm + n_pieces;
-  uint64_t gx = std::min<uint64_t>(n_wg, std::max<uint64_t>(1ull << 16, (n_wg + kMaxGridY - 1) / kMaxGridY));
-  if (gx < n_wg) gx = (gx + 7) / 8 * 8;
-  if (gx > 0xffffffffull / L) return fail(EMRS_ERR_INVALID_ARGUMENT, "plan has too many chunks for one launch");
-  const dim3 grid((uint32_t)gx, (uint32_t)((n_wg + gx - 1) / gx));
+  dim3 grid;
+  if (!tight_grid(n_warm + n_pieces, L, &grid))
+    return fail(EMRS_ERR_INVALID_ARGUMENT, "plan has too many chunks for one launch");
   if (c.nt && c.rb->table) launch_kernel<true, true, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
   else if (c.nt) launch_kernel<true, false, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
   else if (c.rb->table) launch_kernel<false, true, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
