@@ -2182,10 +2182,10 @@ int emrs_plan_create(const emrs_segment *segs, uint64_t n_segs, const uint64_t *
     bld.vec_bytes += all16 ? L : (together ? (L - head) / 16 * 16 : 0);
     bld.scalar_bytes += all16 ? 0 : (together ? L - (L - head) / 16 * 16 : L);
     // Row units (see kRowUnits) wherever 16-byte units do not fit.  Where they
-    // do fit they stay, on lines or not: row units gained 0-1% on segments off
-    // the lines of large plans, but cost 8% on the tiny model's TP2 -> TP1 switch
-    // and 7% on a 1.9 GB one.  Byte elements stay on the element path: no tensor
-    // of a training state has them.
+    // do fit they stay, on lines or not: row units for segments off the lines
+    // gained 0-1% on switches of 9 GB and more, but cost 2% and 5% on ones of 0.9
+    // and 4 GB.  Byte elements stay on the element path: no tensor of a training
+    // state has them.
     const bool by_rows = lg > 0 && !all16 && run >= 16;
     const uint32_t ul = by_rows ? (uint32_t)lg : (all16 ? 4u : (uint32_t)lg);
     const uint64_t ub = 1ull << ul, aub = has_aux ? ub * aeb / eb : 1;  // bytes per unit, and per aux unit
