@@ -257,6 +257,27 @@ __device__ __forceinline__ void copy_chunk(const DevSeg &s, const char *sbase, c
 // Units at any multiple of 2 bytes (the hardware takes them, and the compiler emits whole loads and stores).
 typedef u32x4 __attribute__((aligned(2))) u32x4_any;
 typedef CastOf<u32x4>::type __attribute__((aligned(2))) u32x2_any;
+// Accesses to them of their own: as a template argument the type would lose its alignment.
+template <bool kNT>
+__device__ __forceinline__ u32x4 ld16(const char *p) {
+  if constexpr (kNT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any *>(p));
+  else return *reinterpret_cast<const u32x4_any *>(p);
+}
+template <bool kNT>
+__device__ __forceinline__ CastOf<u32x4>::type ld8(const char *p) {
+  if constexpr (kNT) return __builtin_nontemporal_load(reinterpret_cast<const u32x2_any *>(p));
+  else return *reinterpret_cast<const u32x2_any *>(p);
+}
+template <bool kNT>
+__device__ __forceinline__ void st16(char *p, u32x4 v) {
+  if constexpr (kNT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any *>(p));
+  else *reinterpret_cast<u32x4_any *>(p) = v;
+}
+template <bool kNT>
+__device__ __forceinline__ void st8(char *p, CastOf<u32x4>::type v) {
+  if constexpr (kNT) __builtin_nontemporal_store(v, reinterpret_cast<u32x2_any *>(p));
+  else *reinterpret_cast<u32x2_any *>(p) = v;
+}
 
 // Row units [u0, u0 + L * U) of segment s (clipped to u_end) by a workgroup of
 // L lanes, U units per lane, every load issued before the first store.
@@ -270,17 +291,17 @@ __device__ __forceinline__ void copy_rows(const DevSeg &s, const char *sbase, ch
     v[j] = u32x4{};
     if constexpr (!kZero) {
       const RowUnit r = row_unit(s, dbase, u0 + j * L + threadIdx.x, u_end);
-      if (r.on) v[j] = ld<u32x4_any, kNT>(reinterpret_cast<const u32x4_any *>(sbase + (r.src << lg)));
+      if (r.on) v[j] = ld16<kNT>(sbase + (r.src << lg));
     }
   }
 #pragma unroll
   for (int j = 0; j < U; ++j) {
     const RowUnit r = row_unit(s, dbase, u0 + j * L + threadIdx.x, u_end);
     if (r.on) {
-      st<u32x4_any, kNT>(reinterpret_cast<u32x4_any *>(dbase + (r.dst << lg)), v[j]);
+      st16<kNT>(dbase + (r.dst << lg), v[j]);
       if constexpr (kCast)
-        st<u32x2_any, kNT>(reinterpret_cast<u32x2_any *>(abase + (r.aux << 1)), CastOf<u32x4>::cast(v[j]));
-      if constexpr (kDup) st<u32x4_any, kNT>(reinterpret_cast<u32x4_any *>(abase + (r.aux << lg)), v[j]);
+        st8<kNT>(abase + (r.aux << 1), CastOf<u32x4>::cast(v[j]));
+      if constexpr (kDup) st16<kNT>(abase + (r.aux << lg), v[j]);
     }
   }
 }
@@ -1489,19 +1510,19 @@ __device__ __forceinline__ void compare_rows(const DevSeg &s, const char *sbase,
     const RowUnit r = row_unit(s, dbase, u0 + j * kThreads + threadIdx.x, u_end);
     if (!r.on) continue;
     u32x4 e = u32x4{};
-    if (!(ops & 2)) e = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(sbase + (r.src << lg)));
-    const u32x4 g = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(dbase + (r.dst << lg)));
+    if (!(ops & 2)) e = ld16<true>(sbase + (r.src << lg));
+    const u32x4 g = ld16<true>(dbase + (r.dst << lg));
     uint32_t ew[4], gw[4];
     words_of(e, ew);
     words_of(g, gw);
     cmp_words(m, ew, gw, 16, lg, r.first, r.last);
     if (ops & 4) {
-      const u32x4 d = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(abase + (r.aux << lg)));
+      const u32x4 d = ld16<true>(abase + (r.aux << lg));
       words_of(d, gw);
       cmp_words(x, ew, gw, 16, lg, r.first, r.last);
     }
     if (ops & 1) {
-      const CastOf<u32x4>::type a = ld<u32x2_any, true>(reinterpret_cast<const u32x2_any *>(abase + (r.aux << 1)));
+      const CastOf<u32x4>::type a = ld8<true>(abase + (r.aux << 1));
       uint32_t ea[2], ga[2];
       aux_words_of(CastOf<u32x4>::cast(e), ea);
       aux_words_of(a, ga);
@@ -1623,8 +1644,8 @@ __device__ __forceinline__ void differ_rows(const DevSeg &s, const char *sbase, 
     const RowUnit r = row_unit(s, dbase, u0 + j * L + threadIdx.x, u_end);
     e[j] = g[j] = u32x4{};
     if (r.on) {
-      if (!(ops & 2)) e[j] = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(sbase + (r.src << lg)));
-      g[j] = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(dbase + (r.dst << lg)));
+      if (!(ops & 2)) e[j] = ld16<true>(sbase + (r.src << lg));
+      g[j] = ld16<true>(dbase + (r.dst << lg));
     }
   }
 #pragma unroll
@@ -1634,10 +1655,10 @@ __device__ __forceinline__ void differ_rows(const DevSeg &s, const char *sbase, 
     const RowUnit r = row_unit(s, dbase, u0 + j * L + threadIdx.x, u_end);
     if (!r.on) continue;
     if (ops & 4) {
-      const u32x4 d = ld<u32x4_any, true>(reinterpret_cast<const u32x4_any *>(abase + (r.aux << lg)));
+      const u32x4 d = ld16<true>(abase + (r.aux << lg));
       dx |= differ(e[j], d);
     } else {
-      const CastOf<u32x4>::type a = ld<u32x2_any, true>(reinterpret_cast<const u32x2_any *>(abase + (r.aux << 1)));
+      const CastOf<u32x4>::type a = ld8<true>(abase + (r.aux << 1));
       dx |= differ(CastOf<u32x4>::cast(e[j]), a);
     }
   }
