@@ -95,6 +95,11 @@ constexpr uint64_t kMaxGridY = 65535;                     // rows of a one-workg
 // it cost 5.8% and 1.4%, the launch being too short for per-XCD windows.
 constexpr uint64_t kXcdRemapMinChunks = 1ull << 19;
 constexpr uint64_t kMaxUnitsPerSeg = 1ull << 30;       // keeps unit math in 32 bits
+// Units per lane of a comparison's first pass.  Same allocations, calls of 4 / 2
+// / 1 units: 9.2 GB in short rows 1375 / 1338 / 1335 us, 28 GB 4004 / 3975 /
+// 4047, 42 GB 5585 / 5588 / 5655, 44 GB 6414 / 6412 / 6484: two read as much as
+// they wait for and leave no lane of a short segment idle.
+constexpr int kDifferUnits = 2;
 constexpr int kDifferBlocksPerCu = 4;                  // workgroups per CU of a comparison's first pass
 // Row pitches of multi-row segments stay below this many bytes, so that a piece
 // of at most 256 rows spans less than 2^31 bytes from its first row: the
@@ -906,6 +911,8 @@ struct emrs_plan {
   // reused once its launch has finished).  Destroying the plan frees its tables in stream order
   // after these launches, and waits for nothing else.
   std::vector<std::vector<hipEvent_t>> launch_events;
+  // Per device: the flags of a comparison's first pass, all zero, between two comparisons.
+  std::vector<uint32_t *> differ_flags;
   bool captured = false;  // a launch was recorded into a graph: destroy drains the device first
 };
 
@@ -1580,56 +1587,82 @@ __device__ __forceinline__ void differ_chunk(const DevSeg &s, const char *sbase,
   }
 }
 
-// First pass of a comparison on the copy kernel's schedule: one 64-lane
-// workgroup per piece of U units of a chunk (U = 4: one workgroup per 4 KB
-// chunk), its segment from the plan's chunk table, dispatched in order and,
-// on large plans, each XCD on its own eighth of the pieces.  Every lane issues
-// its U units' source and destination loads before it compares them.  Faster
-// than the persistent grid on every full-size switch (2-4%, same allocations):
-// a segment's rows or gathered runs are spread over many workgroups in flight.
-template <typename T, int U>
+// The bit-level pass over units [u0, u0 + 64 * U) of segment s (clipped to its
+// `total` units) by one wave.  Every lane issues all its units' loads, the
+// second destination's (kAux: 1 a bf16 image, 2 a duplicate) among them, before
+// it compares: one round trip to HBM per workgroup.
+template <typename T, int U, int kAux>
 __device__ __forceinline__ void differ_units(const DevSeg &s, const char *sbase, const char *dbase,
                                              const char *abase, uint32_t u0, uint32_t total, uint32_t &dm,
                                              uint32_t &dx) {
-  typedef typename std::conditional<sizeof(T) == 16 || sizeof(T) == 4, CastOf<T>, CastOf<uint32_t>>::type C;
-  typedef typename C::type A;
+  typedef typename std::conditional<kAux == 1, CastOf<T>, CastOf<uint32_t>>::type C;
+  typedef typename std::conditional<kAux == 1, typename C::type, T>::type X;
   const T *src = reinterpret_cast<const T *>(sbase);
   const T *dst = reinterpret_cast<const T *>(dbase);
-  const A *aux = reinterpret_cast<const A *>(abase);
-  const T *dup = reinterpret_cast<const T *>(abase);
-  const uint32_t ops = s.ops();
+  const X *aux = reinterpret_cast<const X *>(abase);
+  const bool zero = (s.ops() & 2) != 0;
   T e[U], g[U];
-  uint64_t ao[U];
+  X x[U];
 #pragma unroll
   for (int j = 0; j < U; ++j) {
     const uint32_t u = u0 + j * 64 + threadIdx.x;
     e[j] = T{};
     g[j] = T{};
-    ao[j] = 0;
+    x[j] = X{};
     if (u < total) {
-      uint64_t so = s.src_off + u, dof = s.dst_off + u;
-      ao[j] = s.aux_off + u;
+      uint64_t so = s.src_off + u, dof = s.dst_off + u, ao = s.aux_off + u;
       if (s.rows > 1) {
         const uint32_t row = magic_div(u, s.magic, s.sh1(), s.sh2()), col = u - row * s.len;
         so = s.src_off + (uint64_t)row * s.src_stride + col;
         dof = s.dst_off + (uint64_t)row * s.dst_stride + col;
-        ao[j] = s.aux_off + (uint64_t)row * s.aux_stride + col;
+        ao = s.aux_off + (uint64_t)row * s.aux_stride + col;
       }
-      if (!(ops & 2)) e[j] = ld<T, true>(src + so);
+      if (!zero) e[j] = ld<T, true>(src + so);
       g[j] = ld<T, true>(dst + dof);
+      if constexpr (kAux != 0) x[j] = ld<X, true>(aux + ao);
     }
   }
+  // Units past the end are zero on every side, and so is the image of zero.
 #pragma unroll
   for (int j = 0; j < U; ++j) {
-    const uint32_t u = u0 + j * 64 + threadIdx.x;
-    if (u < total) {
-      dm |= differ(e[j], g[j]);
-      if (ops & 4) dx |= differ(e[j], ld<T, true>(dup + ao[j]));
-      if constexpr (sizeof(T) == 16 || sizeof(T) == 4) {
-        if (ops & 1) dx |= differ(C::cast(e[j]), ld<A, true>(aux + ao[j]));
-      }
+    dm |= differ(e[j], g[j]);
+    if constexpr (kAux == 1) dx |= differ(C::cast(e[j]), x[j]);
+    if constexpr (kAux == 2) dx |= differ(e[j], x[j]);
+  }
+}
+
+// differ_units for the segment's second destination, if it has one.
+template <typename T, int U>
+__device__ __forceinline__ void dispatch_differ(const DevSeg &s, const char *sb, const char *db, const char *ab,
+                                                uint32_t u0, uint32_t total, uint32_t &dm, uint32_t &dx) {
+  const uint32_t ops = s.ops();
+  if (ops & 4) {
+    differ_units<T, U, 2>(s, sb, db, ab, u0, total, dm, dx);
+    return;
+  }
+  if constexpr (sizeof(T) == 16 || sizeof(T) == 4) {
+    if (ops & 1) {
+      differ_units<T, U, 1>(s, sb, db, ab, u0, total, dm, dx);
+      return;
     }
   }
+  differ_units<T, U, 0>(s, sb, db, ab, u0, total, dm, dx);
+}
+
+// What a comparison's first pass finds: per device segment, bit 0 where its
+// destination differs and bit 1 where its second destination does; and, if
+// `any` is not null, a word of host memory set once something differs.
+struct DifferMarks {
+  uint32_t *flags;
+  uint32_t *any;
+};
+
+// Mark a segment that differs; one lane per wave that saw a difference calls it.  Nothing is written
+// where the segment is marked already, so that a destination that differs all over stays cheap.
+__device__ __forceinline__ void mark_segment(const DifferMarks &m, uint32_t seg, uint32_t bits) {
+  if ((__hip_atomic_load(m.flags + seg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bits) == bits) return;
+  atomicOr(m.flags + seg, bits);
+  if (m.any) __hip_atomic_store(m.any, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The bit-level pass over row units [u0, u0 + L * U) (clipped to u_end), every
@@ -1664,65 +1697,74 @@ __device__ __forceinline__ void differ_rows(const DevSeg &s, const char *sbase, 
   }
 }
 
-template <bool kTable, int U>
+// First pass of a comparison on the copy kernel's schedule and with its short
+// chain of scalar loads (see copy_pieces_kernel): the first workgroups read the
+// tables, then one 64-lane workgroup per piece of U units a lane takes its
+// segment from the plan's chunk table, dispatched in order and, on large plans,
+// each XCD on its own eighth of the pieces.  Faster than the persistent grid on
+// every full-size switch (2-4%, same allocations): a segment's rows or gathered
+// runs are spread over many workgroups in flight.  Bound by reading HBM.  Whole
+// calls before the pre-read, the preloaded arguments, two units a lane and the
+// marks in place of accumulators, and with them (one process, same
+// allocations): 1 MB 52 and 31 us, 1.0 GB 194 and 174, 9.2 GB in short rows
+// 1567 and 1338, 28 GB 4016 and 3975, 44 GB 6437 and 6412.
+template <bool kTable, int U, typename B>
 __global__ __launch_bounds__(64) void differ_piece_kernel(
-    const DevSeg *__restrict__ segs, uint64_t n_chunks, Bases src, Bases dst, const uint64_t *__restrict__ src_tab,
-    const uint64_t *__restrict__ dst_tab, uint64_t xcd_share, const uint32_t *__restrict__ chunk_seg,
-    const uint32_t *__restrict__ groups, const uint32_t *__restrict__ aux_groups, GroupAcc *__restrict__ acc) {
+    const uint32_t *__restrict__ chunk_seg, const DevSeg *__restrict__ segs, uint64_t n_chunks, uint64_t xcd_share,
+    uint32_t gx, uint32_t n_warm, const uint64_t *__restrict__ src_tab, const uint64_t *__restrict__ dst_tab, B src,
+    B dst, uint32_t n_segs, DifferMarks marks) {
   constexpr uint32_t kPieces = kChunkUnits / (64 * U);
-  uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  uint64_t w = (uint64_t)blockIdx.y * gx + blockIdx.x;
+  if (w < n_warm) {
+    warm_tables<64>(chunk_seg, segs, n_chunks, n_segs, (uint32_t)w);
+    return;
+  }
+  w -= n_warm;
   if (w < xcd_share * 8) w = (w & 7) * xcd_share + (w >> 3);
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;
   const uint32_t lo = chunk_seg[c];
-  const DevSeg s = segs[lo];
+  const DevSeg s = load_seg(segs + lo);
   const uint32_t total = s.units();
   const uint32_t u0 = (uint32_t)(c - s.chunk_begin) * kChunkUnits + (uint32_t)(w % kPieces) * (64 * U);
-  if (kPieces > 1 && u0 >= total) return;
   const char *sb = base_of<kTable>(src, src_tab, s.src_buf());
   const char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
   const char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
+  if (kPieces > 1 && u0 >= total) return;
   uint32_t dm = 0, dx = 0;
   switch (s.unit_log2()) {
     case kRowUnits: differ_rows<64, U>(s, sb, db, ab, u0, total, dm, dx); break;
-    case 4: differ_units<u32x4, U>(s, sb, db, ab, u0, total, dm, dx); break;
-    case 3: differ_units<uint64_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
-    case 2: differ_units<uint32_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
-    case 1: differ_units<uint16_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
-    default: differ_units<uint8_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
+    case 4: dispatch_differ<u32x4, U>(s, sb, db, ab, u0, total, dm, dx); break;
+    case 3: dispatch_differ<uint64_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
+    case 2: dispatch_differ<uint32_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
+    case 1: dispatch_differ<uint16_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
+    default: dispatch_differ<uint8_t, U>(s, sb, db, ab, u0, total, dm, dx); break;
   }
-  if (__any(dm != 0) && threadIdx.x == 0) atomicOr(&acc[groups[lo]].mismatches, 1ull);
-  if ((s.ops() & 5) && __any(dx != 0) && threadIdx.x == 0) atomicOr(&acc[aux_groups[lo]].mismatches, 1ull);
-}
-
-// Mark the groups whose elements differ: one atomic per wave that saw a
-// difference, none for a wave that saw none.  No barrier: each wave marks on
-// its own.
-__device__ __forceinline__ void mark_differ(uint32_t &dm, uint32_t &dx, uint32_t g, uint32_t ga, bool aux,
-                                            GroupAcc *acc) {
-  const bool lead = (threadIdx.x & 63) == 0;
-  if (__any(dm != 0) && lead) atomicOr(&acc[g].mismatches, 1ull);
-  if (aux && __any(dx != 0) && lead) atomicOr(&acc[ga].mismatches, 1ull);
-  dm = dx = 0;
+  const uint32_t bits = (__any(dm != 0) ? 1u : 0u) | (__any(dx != 0) ? 2u : 0u);
+  if (bits && threadIdx.x == 0) mark_segment(marks, lo, bits);
 }
 
 // First pass of a comparison when the plan has no chunk table on the device
 // (it did not fit, or emrs_plan_compare_static meets a plan that has never
-// run there): which groups differ at all, on compare_plan_kernel's persistent
+// run there): which segments differ at all, on compare_plan_kernel's persistent
 // schedule.  Per lane only two words of differing bits are kept.  Only the
-// groups it marks are compared again for compare_ckpt's figures
+// groups of the segments it marks are compared again for compare_ckpt's figures
 // (compare_plan_kernel), whose per-element fp64 work costs about 4% more time
 // on Llama-2-7B than reading alone.
 template <bool kTable>
 __global__ __launch_bounds__(kThreads) void differ_plan_kernel(
-    const DevSeg *__restrict__ segs, const uint32_t *__restrict__ groups, const uint32_t *__restrict__ aux_groups,
-    uint32_t n_segs, uint64_t n_chunks, uint32_t run, Bases src, Bases dst, const uint64_t *__restrict__ src_tab,
-    const uint64_t *__restrict__ dst_tab, GroupAcc *__restrict__ acc) {
+    const DevSeg *__restrict__ segs, uint32_t n_segs, uint64_t n_chunks, uint32_t run, Bases src, Bases dst,
+    const uint64_t *__restrict__ src_tab, const uint64_t *__restrict__ dst_tab, DifferMarks marks) {
   const uint64_t xcd = blockIdx.x & 7;
   const uint64_t c1 = n_chunks * (xcd + 1) / 8;
   const uint64_t step = (uint64_t)(gridDim.x >> 3) * run;
-  uint32_t dm = 0, dx = 0, cur_g = 0, cur_ga = 0;
-  bool open = false, cur_aux = false;
+  uint32_t dm = 0, dx = 0, cur = 0;
+  // Each wave marks on its own: no barrier.
+  auto mark = [&](uint32_t seg) {
+    const uint32_t bits = (__any(dm != 0) ? 1u : 0u) | (__any(dx != 0) ? 2u : 0u);
+    if (bits && (threadIdx.x & 63) == 0) mark_segment(marks, seg, bits);
+    dm = dx = 0;
+  };
   for (uint64_t c = n_chunks * xcd / 8 + (uint64_t)(blockIdx.x >> 3) * run; c < c1; c += step) {
     const uint64_t c_end = min(c + run, c1);
     uint32_t lo = 0, hi = n_segs - 1;
@@ -1740,13 +1782,8 @@ __global__ __launch_bounds__(kThreads) void differ_plan_kernel(
       }
       nq = min(min(c_end, s_end) - q, (uint64_t)kUnroll);
       const DevSeg s = segs[si];
-      const uint32_t g = groups[si], ga = aux_groups[si];
-      const bool aux = (s.ops() & 5) != 0;
-      if (open && (g != cur_g || aux != cur_aux || (aux && ga != cur_ga))) mark_differ(dm, dx, cur_g, cur_ga, cur_aux, acc);
-      open = true;
-      cur_g = g;
-      cur_ga = ga;
-      cur_aux = aux;
+      if (si != cur) mark(cur);
+      cur = si;
       const uint32_t total = s.units();
       const uint32_t u0 = (uint32_t)(q - s.chunk_begin) * kChunkUnits;
       const uint32_t u_end = min(u0 + (uint32_t)nq * kChunkUnits, total);
@@ -1763,7 +1800,7 @@ __global__ __launch_bounds__(kThreads) void differ_plan_kernel(
       }
     }
   }
-  if (open) mark_differ(dm, dx, cur_g, cur_ga, cur_aux, acc);
+  mark(cur);
 }
 
 // Sum / max over the workgroup; the result is valid in thread 0.
@@ -1918,15 +1955,43 @@ bool tight_grid(uint64_t n_wg, uint32_t lanes, dim3 *grid) {
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-// What both comparison entry points prepare on the host: checked bases, the
-// groups of every device segment, and the element counts per group.
+// Workgroups that read a plan's tables ahead of the pieces, a multiple of 8 so that the pieces keep their XCDs.
+uint32_t warm_groups(uint64_t n_chunks, uint64_t n_segs, uint32_t lanes) {
+  const uint64_t units = n_chunks / 4 + n_segs * (sizeof(DevSeg) / sizeof(u32x4));
+  const uint64_t n = ((units + kWarmUnits * lanes - 1) / (kWarmUnits * lanes) + 7) / 8 * 8;
+  return n > 0xffffffffull ? 0 : (uint32_t)n;
+}
+
+// What both comparison entry points prepare on the host: checked bases and the
+// element counts per group.
 struct CompareJob {
   ResolvedBases rb;
-  std::vector<uint32_t> g_host;  // per device segment: its group, then its aux group
+  const uint32_t *groups = nullptr, *aux_groups = nullptr;  // the caller's, one per input segment, or null
   int cus = 0;
-  int resident = 0;              // compare_plan_kernel workgroups per CU
-  int resident_differ = 0;       // differ_plan_kernel workgroups per CU
   const uint32_t *cseg = nullptr;  // the plan's chunk table on this device, if there is one
+
+  // Group of device segment k's destination, and of its second destination.
+  uint32_t group(const emrs_plan *plan, size_t k) const { return groups ? groups[plan->origin[k]] : 0; }
+  uint32_t aux_group(const emrs_plan *plan, size_t k) const {
+    return aux_groups ? aux_groups[plan->origin[k]] : group(plan, k);
+  }
+  // Per device segment its group, then its aux group.
+  std::vector<uint32_t> group_table(const emrs_plan *plan) const {
+    const size_t nd = plan->segs.size();
+    std::vector<uint32_t> t(2 * nd);
+    for (size_t k = 0; k < nd; ++k) t[k] = group(plan, k), t[nd + k] = aux_group(plan, k);
+    return t;
+  }
+  // The groups that the first pass's flags mark; false when there is none.
+  bool marked_groups(const emrs_plan *plan, const std::vector<uint32_t> &flags, std::vector<uint8_t> *mark) const {
+    bool any = false;
+    for (size_t k = 0; k < flags.size(); ++k) {
+      if (flags[k] & 1u) (*mark)[group(plan, k)] = 1;
+      if (flags[k] & 2u) (*mark)[aux_group(plan, k)] = 1;
+      any = any || flags[k];
+    }
+    return any;
+  }
 };
 
 int compare_setup(emrs_plan *plan, void *const *src_bases, void *const *dst_bases, const uint32_t *groups,
@@ -1939,18 +2004,14 @@ int compare_setup(emrs_plan *plan, void *const *src_bases, void *const *dst_base
       return fail(EMRS_ERR_INVALID_ARGUMENT, "group id >= n_groups");
   int rc = resolve_bases(plan, src_bases, dst_bases, &job->rb, /*out_of_place=*/false);
   if (rc) return rc;
-  const size_t nd = plan->segs.size();
-  job->g_host.resize(2 * nd);
+  job->groups = groups;
+  job->aux_groups = aux_groups;
   std::vector<uint64_t> elements(n_groups, 0);
-  for (size_t k = 0; k < nd; ++k) {
+  for (size_t k = 0; k < plan->segs.size(); ++k) {
     const DevSeg &d = plan->segs[k];
-    const uint32_t o = plan->origin[k];
-    const uint32_t g = groups ? groups[o] : 0, ga = aux_groups ? aux_groups[o] : g;
-    job->g_host[k] = g;
-    job->g_host[nd + k] = ga;
     const uint64_t n = ((uint64_t)d.len * d.rows) << (d.off_log2() - d.elem_log2());
-    elements[g] += n;
-    if (d.ops() & 5) elements[ga] += n;
+    elements[job->group(plan, k)] += n;
+    if (d.ops() & 5) elements[job->aux_group(plan, k)] += n;
   }
   for (uint32_t g = 0; g < n_groups; ++g) {
     stats[g] = emrs_compare_stats{};
@@ -1959,109 +2020,185 @@ int compare_setup(emrs_plan *plan, void *const *src_bases, void *const *dst_base
   return EMRS_OK;
 }
 
-// The current device, its CU count and the compare kernel's residency.
+// The current device and its CU count.
 int compare_device(CompareJob *job, int *dev) {
   int resident_nt = 0, resident_t = 0;
-  int rc = current_device(dev, &job->cus, &resident_nt, &resident_t);
-  if (rc) return rc;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&job->resident, compare_plan_kernel<false>, kThreads, 0) !=
-          hipSuccess ||
-      job->resident <= 0) {
+  return current_device(dev, &job->cus, &resident_nt, &resident_t);
+}
+
+// Workgroups per CU that a persistent comparison kernel can hold.
+template <typename K>
+int resident_of(K kernel) {
+  int v = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kernel, kThreads, 0) != hipSuccess || v <= 0) {
     (void)hipGetLastError();
-    job->resident = 4;
+    v = 4;
   }
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&job->resident_differ, differ_plan_kernel<false>, kThreads, 0) !=
-          hipSuccess ||
-      job->resident_differ <= 0) {
-    (void)hipGetLastError();
-    job->resident_differ = job->resident;
-  }
-  return EMRS_OK;
+  return v;
 }
 
 // A persistent grid of resident workgroups, a multiple of 8 (one eighth of
 // the plan per XCD), in runs of up to 32 steps: at most a quarter of each
-// workgroup's share, so that small plans still spread out.  `active` null:
-// the first pass (differ_piece_kernel with the plan's chunk table, else
-// differ_plan_kernel); else the second (compare_plan_kernel).
-hipError_t compare_launch(const emrs_plan *plan, const CompareJob &job, const DevSeg *table, const uint32_t *grp,
-                          const uint64_t *tab, GroupAcc *acc, const uint8_t *active, hipStream_t st) {
-  const size_t nd = plan->segs.size();
-  // The first pass could hold 8 workgroups per CU; 3-6 read at the plain read rate and 8 is up to
-  // 7% slower (Llama-2-7B, Mixtral and Group-ZeRO switches, same allocations): 4.
-  const uint32_t resident = (uint32_t)(active ? job.resident : std::min(job.resident_differ, kDifferBlocksPerCu));
-  uint64_t blocks = std::min<uint64_t>(plan->n_chunks, (uint64_t)job.cus * resident);
+// workgroup's share, so that small plans still spread out.
+void persistent_grid(const emrs_plan *plan, const CompareJob &job, int per_cu, dim3 *grid, uint32_t *run) {
+  uint64_t blocks = std::min<uint64_t>(plan->n_chunks, (uint64_t)job.cus * per_cu);
   blocks = std::max<uint64_t>(8, blocks / 8 * 8);
-  const uint32_t run =
-      (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(32 * kUnroll, plan->n_chunks / (blocks * 4)));
+  *run = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(32 * kUnroll, plan->n_chunks / (blocks * 4)));
+  *grid = dim3((uint32_t)blocks);
+}
+
+// First pass: marks what differs.  differ_piece_kernel with the plan's chunk table, else differ_plan_kernel.
+hipError_t differ_launch(const emrs_plan *plan, const CompareJob &job, const DevSeg *table, const uint64_t *tab,
+                         const DifferMarks &marks, hipStream_t st) {
+  const uint32_t nd = (uint32_t)plan->segs.size();
   const uint64_t *dtab = tab ? tab + plan->stats.n_src_bufs : nullptr;
-  const dim3 grid((uint32_t)blocks), block(kThreads);
-  if (!active && job.cseg) {  // the first pass on the copy kernel's schedule
-    constexpr int U = 4;
-    const uint64_t n_wg = plan->n_chunks * (kChunkUnits / (64 * U));
-    dim3 pgrid;
-    if (!tight_grid(n_wg, 64, &pgrid)) return hipErrorInvalidConfiguration;
+  if (job.cseg) {
+    constexpr int U = kDifferUnits;
+    const uint64_t n_pieces = plan->n_chunks * (kChunkUnits / (64 * U));
+    const uint32_t n_warm = g_tuning.warm_tables.load() ? warm_groups(plan->n_chunks, nd, 64) : 0;
+    dim3 grid;
+    if (!tight_grid(n_warm + n_pieces, 64, &grid)) return hipErrorInvalidConfiguration;
     const uint32_t remap = g_tuning.xcd_remap.load();
     const bool by_xcd = remap == 2 || (remap == 1 && plan->n_chunks >= kXcdRemapMinChunks);
-    const uint64_t xcd_share = by_xcd ? n_wg / 8 : 0;
+    const uint64_t xcd_share = by_xcd ? n_pieces / 8 : 0;
+    FewBases src{}, dst{};
+    if (!job.rb.table)
+      for (uint32_t i = 0; i < kFewBuffers; ++i) src.p[i] = job.rb.src.p[i], dst.p[i] = job.rb.dst.p[i];
     if (job.rb.table)
-      hipLaunchKernelGGL((differ_piece_kernel<true, U>), pgrid, dim3(64), 0, st, table, plan->n_chunks, job.rb.src,
-                         job.rb.dst, tab, dtab, xcd_share, job.cseg, grp, grp + nd, acc);
+      hipLaunchKernelGGL((differ_piece_kernel<true, U, FewBases>), grid, dim3(64), 0, st, job.cseg, table,
+                         plan->n_chunks, xcd_share, grid.x, n_warm, tab, dtab, src, dst, nd, marks);
+    else if (std::max(plan->stats.n_src_bufs, plan->stats.n_dst_bufs) <= kFewBuffers)
+      hipLaunchKernelGGL((differ_piece_kernel<false, U, FewBases>), grid, dim3(64), 0, st, job.cseg, table,
+                         plan->n_chunks, xcd_share, grid.x, n_warm, tab, dtab, src, dst, nd, marks);
     else
-      hipLaunchKernelGGL((differ_piece_kernel<false, U>), pgrid, dim3(64), 0, st, table, plan->n_chunks, job.rb.src,
-                         job.rb.dst, tab, dtab, xcd_share, job.cseg, grp, grp + nd, acc);
+      hipLaunchKernelGGL((differ_piece_kernel<false, U, Bases>), grid, dim3(64), 0, st, job.cseg, table,
+                         plan->n_chunks, xcd_share, grid.x, n_warm, tab, dtab, job.rb.src, job.rb.dst, nd, marks);
     return hipGetLastError();
   }
-  if (!active) {
-    if (job.rb.table)
-      hipLaunchKernelGGL(differ_plan_kernel<true>, grid, block, 0, st, table, grp, grp + nd, (uint32_t)nd,
-                         plan->n_chunks, run, job.rb.src, job.rb.dst, tab, dtab, acc);
-    else
-      hipLaunchKernelGGL(differ_plan_kernel<false>, grid, block, 0, st, table, grp, grp + nd, (uint32_t)nd,
-                         plan->n_chunks, run, job.rb.src, job.rb.dst, tab, dtab, acc);
-  } else if (job.rb.table) {
-    hipLaunchKernelGGL(compare_plan_kernel<true>, grid, block, 0, st, table, grp, grp + nd, (uint32_t)nd,
-                       plan->n_chunks, run, job.rb.src, job.rb.dst, tab, dtab, acc, active);
-  } else {
-    hipLaunchKernelGGL(compare_plan_kernel<false>, grid, block, 0, st, table, grp, grp + nd, (uint32_t)nd,
-                       plan->n_chunks, run, job.rb.src, job.rb.dst, tab, dtab, acc, active);
-  }
+  // It could hold 8 workgroups per CU; 3-6 read at the plain read rate and 8 is up to
+  // 7% slower (Llama-2-7B, Mixtral and Group-ZeRO switches, same allocations): 4.
+  dim3 grid;
+  uint32_t run = 0;
+  persistent_grid(plan, job, std::min(resident_of(differ_plan_kernel<false>), kDifferBlocksPerCu), &grid, &run);
+  if (job.rb.table)
+    hipLaunchKernelGGL(differ_plan_kernel<true>, grid, dim3(kThreads), 0, st, table, nd, plan->n_chunks, run,
+                       job.rb.src, job.rb.dst, tab, dtab, marks);
+  else
+    hipLaunchKernelGGL(differ_plan_kernel<false>, grid, dim3(kThreads), 0, st, table, nd, plan->n_chunks, run,
+                       job.rb.src, job.rb.dst, tab, dtab, marks);
   return hipGetLastError();
 }
 
-// Zero the accumulators with a kernel (no memset node if the stream's work is ever captured).
-hipError_t clear_acc(GroupAcc *acc, uint32_t n_groups, hipStream_t st) {
-  const uint64_t words = (uint64_t)n_groups * sizeof(GroupAcc) / sizeof(uint32_t);
+// Zero 32-bit words with a kernel (no memset node if the stream's work is ever captured).
+hipError_t clear_words(void *p, uint64_t words, hipStream_t st) {
   hipLaunchKernelGGL(clear_words_kernel, dim3((uint32_t)std::min<uint64_t>(1024, (words + 255) / 256)), dim3(256), 0,
-                     st, reinterpret_cast<uint32_t *>(acc), words);
+                     st, static_cast<uint32_t *>(p), words);
   return hipGetLastError();
 }
 
-// Both passes of a comparison, on device buffers the caller provides (acc:
-// n_groups accumulators; active: n_groups bytes), leaving the accumulators
-// in `host`.  The first pass marks the groups that differ in any bit; when
-// none does (a correct switch), every figure is 0 and the second pass does
-// not run.  Otherwise the marked groups are compared again with every figure.
-hipError_t compare_passes(const emrs_plan *plan, const CompareJob &job, const DevSeg *table, const uint32_t *grp,
-                          const uint64_t *tab, GroupAcc *acc, uint8_t *active, uint32_t n_groups, hipStream_t st,
-                          std::vector<GroupAcc> &host) {
-  const size_t acc_bytes = (size_t)n_groups * sizeof(GroupAcc);
-  hipError_t e = clear_acc(acc, n_groups, st);
-  if (e == hipSuccess) e = compare_launch(plan, job, table, grp, tab, acc, nullptr, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(host.data(), acc, acc_bytes, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (e != hipSuccess) return e;
-  std::vector<uint8_t> mark(n_groups, 0);
-  bool any = false;
-  for (uint32_t g = 0; g < n_groups; ++g)
-    if (host[g].mismatches) mark[g] = 1, any = true;
-  if (!any) return hipSuccess;
-  e = hipMemcpyAsync(active, mark.data(), n_groups, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = clear_acc(acc, n_groups, st);
-  if (e == hipSuccess) e = compare_launch(plan, job, table, grp, tab, acc, active, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(host.data(), acc, acc_bytes, hipMemcpyDeviceToHost, st);
-  const hipError_t se = hipStreamSynchronize(st);  // `mark` is read by the copy above
+// Second pass of a comparison, when the first has marked groups: every figure
+// of those, on device buffers the caller provides (acc: n_groups accumulators;
+// grp: two group ids per device segment; active: n_groups bytes), leaving the
+// accumulators in `host`.  Waits for the stream: `mark` and the group table
+// are read by the copies.
+hipError_t compare_marked(const emrs_plan *plan, const CompareJob &job, const DevSeg *table, uint32_t *grp,
+                          const uint64_t *tab, GroupAcc *acc, uint8_t *active, const std::vector<uint8_t> &mark,
+                          hipStream_t st, std::vector<GroupAcc> &host) {
+  const uint32_t nd = (uint32_t)plan->segs.size();
+  const uint64_t *dtab = tab ? tab + plan->stats.n_src_bufs : nullptr;
+  const std::vector<uint32_t> gt = job.group_table(plan);
+  dim3 grid;
+  uint32_t run = 0;
+  persistent_grid(plan, job, resident_of(compare_plan_kernel<false>), &grid, &run);
+  hipError_t e = hipMemcpyAsync(grp, gt.data(), gt.size() * sizeof(uint32_t), hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(active, mark.data(), mark.size(), hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = clear_words(acc, host.size() * sizeof(GroupAcc) / sizeof(uint32_t), st);
+  if (e == hipSuccess) {
+    if (job.rb.table)
+      hipLaunchKernelGGL(compare_plan_kernel<true>, grid, dim3(kThreads), 0, st, table, grp, grp + nd, nd,
+                         plan->n_chunks, run, job.rb.src, job.rb.dst, tab, dtab, acc, active);
+    else
+      hipLaunchKernelGGL(compare_plan_kernel<false>, grid, dim3(kThreads), 0, st, table, grp, grp + nd, nd,
+                         plan->n_chunks, run, job.rb.src, job.rb.dst, tab, dtab, acc, active);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(host.data(), acc, host.size() * sizeof(GroupAcc), hipMemcpyDeviceToHost, st);
+  const hipError_t se = hipStreamSynchronize(st);
   return e == hipSuccess ? se : e;
+}
+
+// Words of pinned host memory that comparisons in flight are told a difference
+// through: one page for the process, one 64-byte slot per comparison.  Null
+// when all are in use or the page could not be made: the comparison then
+// reads its flags back.
+struct AnySlots {
+  static constexpr int kSlots = 64;
+  std::mutex mu;
+  uint32_t *page = nullptr;
+  bool tried = false;
+  uint64_t used = 0;
+};
+AnySlots g_any;
+
+uint32_t *take_any_slot() {
+  std::lock_guard<std::mutex> lk(g_any.mu);
+  if (!g_any.tried) {
+    g_any.tried = true;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, AnySlots::kSlots * 64,
+                      hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess)
+      g_any.page = static_cast<uint32_t *>(p);
+    else
+      (void)hipGetLastError();
+  }
+  if (!g_any.page) return nullptr;
+  for (int i = 0; i < AnySlots::kSlots; ++i)
+    if (!((g_any.used >> i) & 1u)) {
+      g_any.used |= 1ull << i;
+      return g_any.page + i * 16;
+    }
+  return nullptr;
+}
+
+void give_any_slot(uint32_t *slot) {
+  if (!slot) return;
+  std::lock_guard<std::mutex> lk(g_any.mu);
+  g_any.used &= ~(1ull << ((slot - g_any.page) / 16));
+}
+
+// The plan's flags on device `dev`, all zero: one array is kept between
+// comparisons (a comparison has waited for its stream when it gives the array
+// back, and has cleared what it marked), and concurrent ones get arrays of
+// their own.
+int take_flags(emrs_plan *plan, int dev, hipStream_t st, uint32_t **out) {
+  {
+    std::lock_guard<std::mutex> lk(plan->mu);
+    if ((int)plan->differ_flags.size() <= dev) plan->differ_flags.resize(dev + 1, nullptr);
+    *out = plan->differ_flags[dev];
+    plan->differ_flags[dev] = nullptr;
+  }
+  if (*out) return EMRS_OK;
+  const uint64_t nd = plan->segs.size();
+  hipError_t e = table_alloc(reinterpret_cast<void **>(out), nd * sizeof(uint32_t), st);
+  if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(compare flags)");
+  e = clear_words(*out, nd, st);
+  if (e == hipSuccess) return EMRS_OK;
+  (void)hipFreeAsync(*out, st);
+  *out = nullptr;
+  return hip_fail(e, "clearing the compare flags");
+}
+
+// `clean`: the array is all zero again and no launch uses it.
+void give_flags(emrs_plan *plan, int dev, hipStream_t st, uint32_t *flags, bool clean) {
+  if (clean) {
+    std::lock_guard<std::mutex> lk(plan->mu);
+    if (!plan->differ_flags[dev]) {
+      plan->differ_flags[dev] = flags;
+      return;
+    }
+  }
+  (void)hipFreeAsync(flags, st);
 }
 
 void compare_finish(const std::vector<GroupAcc> &host, emrs_compare_stats *stats) {
@@ -2297,13 +2434,7 @@ int launch_chunks(const CopyLaunch &c) {
   const uint32_t remap = g_tuning.xcd_remap.load();
   const bool by_xcd = remap == 2 || (remap == 1 && c.n_chunks >= kXcdRemapMinChunks);
   const uint64_t xcd_share = by_xcd ? n_pieces / 8 : 0;
-  // Workgroups that read the tables first, a multiple of 8 so that the pieces keep their XCDs.
-  uint64_t n_warm = 0;
-  if (c.cseg && c.warm) {
-    const uint64_t units = c.n_chunks / 4 + (uint64_t)c.n_segs * (sizeof(DevSeg) / sizeof(u32x4));
-    n_warm = ((units + kWarmUnits * L - 1) / (kWarmUnits * L) + 7) / 8 * 8;
-    if (n_warm > 0xffffffffull) n_warm = 0;
-  }
+  const uint64_t n_warm = c.cseg && c.warm ? warm_groups(c.n_chunks, c.n_segs, L) : 0;
   dim3 grid;
   if (!tight_grid(n_warm + n_pieces, L, &grid))
     return fail(EMRS_ERR_INVALID_ARGUMENT, "plan has too many chunks for one launch");
@@ -2479,31 +2610,59 @@ int emrs_plan_compare(emrs_plan *plan, void *const *src_bases, void *const *dst_
   rc = device_table(plan, dev, st, &table);
   if (rc) return rc;
 
-  const size_t acc_bytes = align256((size_t)n_groups * sizeof(GroupAcc));
-  const size_t grp_bytes = align256(job.g_host.size() * sizeof(uint32_t));
-  char *buf = nullptr;
-  hipError_t e = hipMalloc(&buf, acc_bytes + grp_bytes + n_groups);
-  if (e != hipSuccess) return hip_fail(e, "hipMalloc(compare buffers)");
-  GroupAcc *acc = reinterpret_cast<GroupAcc *>(buf);
-  uint32_t *grp = reinterpret_cast<uint32_t *>(buf + acc_bytes);
-  uint8_t *active = reinterpret_cast<uint8_t *>(buf + acc_bytes + grp_bytes);
-  std::vector<GroupAcc> host(n_groups);
-  e = hipMemcpyAsync(grp, job.g_host.data(), job.g_host.size() * sizeof(uint32_t), hipMemcpyHostToDevice, st);
   uint64_t *tab = nullptr;
   bool tab_owned = false;
-  int table_rc = EMRS_OK;  // a pointer-table failure keeps its own message
-  if (e == hipSuccess) table_rc = pointer_table(plan, dev, job.rb, st, &tab, &tab_owned);
-  if (e == hipSuccess && table_rc == EMRS_OK) {
-    uint32_t *cseg = nullptr;  // null when it does not fit: the first pass then runs as a persistent grid
-    table_rc = chunk_table(plan, dev, st, table, &cseg);
-    job.cseg = cseg;
+  rc = pointer_table(plan, dev, job.rb, st, &tab, &tab_owned);
+  if (rc) return rc;
+  uint32_t *cseg = nullptr, *flags = nullptr;  // no chunk table when it does not fit: then a persistent grid
+  rc = chunk_table(plan, dev, st, table, &cseg);
+  if (rc == EMRS_OK) rc = take_flags(plan, dev, st, &flags);
+  if (rc) {
+    if (tab_owned) {
+      (void)hipFreeAsync(tab, st);
+      (void)hipStreamSynchronize(st);  // its upload reads job's vector
+    }
+    return rc;
   }
-  if (e == hipSuccess && table_rc == EMRS_OK)
-    e = compare_passes(plan, job, table, grp, tab, acc, active, n_groups, st, host);
+  job.cseg = cseg;
+
+  // A switch that is correct, the common case, costs one launch and one wait:
+  // no buffer is allocated, uploaded or read back.  A comparison of 1 GB used
+  // to allocate, upload the groups, clear, launch, read back and free.
+  const size_t nd = plan->segs.size();
+  uint32_t *any = take_any_slot();
+  if (any) *static_cast<volatile uint32_t *>(any) = 0;
+  hipError_t e = differ_launch(plan, job, table, tab, DifferMarks{flags, any}, st);
+  const hipError_t se = hipStreamSynchronize(st);
+  if (e == hipSuccess) e = se;
+  const bool marked = any == nullptr || *static_cast<volatile uint32_t *>(any) != 0;
+  give_any_slot(any);
+  std::vector<GroupAcc> host(n_groups);
+  bool clean = e == hipSuccess;
+  if (e == hipSuccess && marked) {
+    std::vector<uint32_t> found(nd);
+    std::vector<uint8_t> mark(n_groups, 0);
+    clean = false;
+    e = hipMemcpyAsync(found.data(), flags, nd * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = clear_words(flags, nd, st);
+    const hipError_t fe = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = fe;
+    clean = e == hipSuccess;
+    if (e == hipSuccess && job.marked_groups(plan, found, &mark)) {
+      const size_t acc_bytes = align256((size_t)n_groups * sizeof(GroupAcc));
+      const size_t grp_bytes = align256(2 * nd * sizeof(uint32_t));
+      char *buf = nullptr;
+      e = hipMalloc(&buf, acc_bytes + grp_bytes + n_groups);
+      if (e == hipSuccess) {
+        e = compare_marked(plan, job, table, reinterpret_cast<uint32_t *>(buf + acc_bytes), tab,
+                           reinterpret_cast<GroupAcc *>(buf), reinterpret_cast<uint8_t *>(buf + acc_bytes + grp_bytes),
+                           mark, st, host);
+        (void)hipFree(buf);
+      }
+    }
+  }
+  give_flags(plan, dev, st, flags, clean);
   if (tab_owned) (void)hipFreeAsync(tab, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  (void)hipFree(buf);
-  if (table_rc != EMRS_OK) return table_rc;
   if (e != hipSuccess) return hip_fail(e, "compare_plan_kernel");
   compare_finish(host, stats);
   return EMRS_OK;
@@ -2520,7 +2679,7 @@ int emrs_plan_compare_static(emrs_plan *plan, void *const *src_bases, void *cons
   // 256-byte aligned regions: accumulators, group ids, the segment table, the pointer table.
   const size_t nd = plan->segs.size();
   const size_t acc_bytes = align256((size_t)n_groups * sizeof(GroupAcc));
-  const size_t grp_bytes = align256(job.g_host.size() * sizeof(uint32_t));
+  const size_t grp_bytes = align256(2 * nd * sizeof(uint32_t));
   const size_t seg_bytes = align256(nd * sizeof(DevSeg));
   const size_t ptr_bytes = job.rb.table ? align256(job.rb.ptrs.size() * sizeof(uint64_t)) : 0;
   const size_t act_bytes = align256(n_groups);
@@ -2550,15 +2709,20 @@ int emrs_plan_compare_static(emrs_plan *plan, void *const *src_bases, void *cons
   DevSeg *table = reinterpret_cast<DevSeg *>(base + acc_bytes + grp_bytes);
   uint64_t *tab = job.rb.table ? reinterpret_cast<uint64_t *>(base + acc_bytes + grp_bytes + seg_bytes) : nullptr;
   uint8_t *active = base + acc_bytes + grp_bytes + seg_bytes + ptr_bytes;
-  // The previous call's accumulators are still there: compare_passes clears them with a kernel.
-  hipError_t e =
-      hipMemcpyAsync(grp, job.g_host.data(), job.g_host.size() * sizeof(uint32_t), hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(table, plan->segs.data(), nd * sizeof(DevSeg), hipMemcpyHostToDevice, st);
+  hipError_t e = hipMemcpyAsync(table, plan->segs.data(), nd * sizeof(DevSeg), hipMemcpyHostToDevice, st);
   if (e == hipSuccess && tab)
     e = hipMemcpyAsync(tab, job.rb.ptrs.data(), job.rb.ptrs.size() * sizeof(uint64_t), hipMemcpyHostToDevice, st);
   std::vector<GroupAcc> host(n_groups);
+  std::vector<uint32_t> found(nd);
+  std::vector<uint8_t> mark(n_groups, 0);
   job.cseg = existing_chunk_table(plan, dev);  // never built here: that would allocate
-  if (e == hipSuccess) e = compare_passes(plan, job, table, grp, tab, acc, active, n_groups, st, host);
+  // The first pass's flags lie where the second pass's group ids go.
+  if (e == hipSuccess) e = clear_words(grp, nd, st);
+  if (e == hipSuccess) e = differ_launch(plan, job, table, tab, DifferMarks{grp, nullptr}, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(found.data(), grp, nd * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e == hipSuccess && job.marked_groups(plan, found, &mark))
+    e = compare_marked(plan, job, table, grp, tab, acc, active, mark, st, host);
   // The host copies above read job's and plan's vectors: wait before they can go.
   const hipError_t se = hipStreamSynchronize(st);
   if (e == hipSuccess) e = se;
@@ -2572,14 +2736,15 @@ int emrs_plan_destroy(emrs_plan *plan) {
   int prev = 0;
   (void)hipGetDevice(&prev);
   const size_t n_dev = std::max({plan->dev_tables.size(), plan->ptr_tables.size(), plan->abs_tables.size(),
-                                  plan->chunk_tables.size(), plan->launch_events.size()});
+                                  plan->chunk_tables.size(), plan->launch_events.size(), plan->differ_flags.size()});
   for (size_t d = 0; d < n_dev; ++d) {
     DevSeg *segs = d < plan->dev_tables.size() ? plan->dev_tables[d] : nullptr;
     uint64_t *ptrs = d < plan->ptr_tables.size() ? plan->ptr_tables[d] : nullptr;
     DevSeg *abs = d < plan->abs_tables.size() ? plan->abs_tables[d] : nullptr;
     uint32_t *chunks = d < plan->chunk_tables.size() ? plan->chunk_tables[d] : nullptr;
     std::vector<hipEvent_t> evs = d < plan->launch_events.size() ? plan->launch_events[d] : std::vector<hipEvent_t>();
-    if (!(segs || ptrs || abs || chunks || !evs.empty())) continue;
+    uint32_t *flags = d < plan->differ_flags.size() ? plan->differ_flags[d] : nullptr;
+    if (!(segs || ptrs || abs || chunks || flags || !evs.empty())) continue;
     (void)hipSetDevice((int)d);
     // A graph may replay the plan's launches at any time: only a drained device is safe.
     if (plan->captured) (void)hipDeviceSynchronize();
@@ -2593,7 +2758,7 @@ int emrs_plan_destroy(emrs_plan *plan) {
     }
     for (hipEvent_t ev : evs) (void)hipEventDestroy(ev);
     for (void *t : {static_cast<void *>(segs), static_cast<void *>(ptrs), static_cast<void *>(abs),
-                    static_cast<void *>(chunks)})
+                    static_cast<void *>(chunks), static_cast<void *>(flags)})
       if (t) (void)hipFreeAsync(t, fs);
   }
   (void)hipSetDevice(prev);
