@@ -178,9 +178,9 @@ def set_tuning(blocks_per_cu: int = 0, nontemporal: bool = True, xcd_remap: int 
     (0: 64) with ``units`` 16-byte units each (0: a whole chunk of 256 units per workgroup) per piece
     of a chunk, each finding its segment in the plan's chunk table (``chunk_index``; False: by a
     bounded binary search); ``persistent=True`` selects a persistent grid, which ``blocks_per_cu``
-    and ``run`` shape.  ``xcd_remap`` gives each of the 8 XCDs one contiguous eighth of the chunks:
-    1 (or True) in the persistent grid and for plans of at least 2^19 chunks, 2 always, 0 (or False)
-    never.  ``warm_tables``: with the chunk table, the first workgroups of each copy launch
+    and ``run`` shape.  ``xcd_remap`` (1, or 2 alike) has each of the 8 XCDs work through runs of
+    consecutive chunks (the persistent grid: through one eighth of them); 0 (or False) keeps the
+    hardware's order.  ``warm_tables``: with the chunk table, the first workgroups of each copy launch
     read it and the segment descriptors, so that a launch after unrelated work starts from cached
     tables."""
     t = Tuning(blocks_per_cu, 1 if nontemporal else 0, int(xcd_remap), run, 1 if persistent else 0, lanes,

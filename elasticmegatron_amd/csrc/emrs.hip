@@ -89,11 +89,21 @@ constexpr int kUnroll = EMRS_COPY_UNROLL;
 constexpr uint32_t kChunkUnits = kThreads;  // units per work chunk: one per lane
 constexpr uint32_t kStepUnits = kThreads * kUnroll;  // units per step of a persistent workgroup
 constexpr uint64_t kMaxGridY = 65535;                     // rows of a one-workgroup-per-chunk grid
-// Plans of at least this many chunks (2 GiB of 16-byte units) give each XCD
-// its own contiguous eighth by default.  Measured on Llama-2-7B-shaped
-// switches: at 0.69M chunks and up it saved 0.3-2%; at 0.11M and 0.24M chunks
-// it cost 5.8% and 1.4%, the launch being too short for per-XCD windows.
-constexpr uint64_t kXcdRemapMinChunks = 1ull << 19;
+// Chunks in a run of one XCD (see xcd_order): 2^8 (1 MB of 16-byte units), and
+// 2^10 in plans of at least 2^19 chunks.  Before, such plans gave each XCD an
+// eighth of all their chunks, and smaller ones kept the hardware's order, which
+// splits neighbouring kilobytes over XCDs: lines and pages at their ends are
+// then fetched by two of them, the more the less aligned the rows are.  us (hardware
+// order, eighths, runs of 2^8, of 2^10), one process, same allocations: 0.1 GB
+// 30.7, 27.0, 29.1, 28.1; 0.55 GB of short rows 107.7, 99.9, 99.4, 99.2; 0.93 GB
+// 164.6, 155.8, 155.4, 155.8; 1.02 GB of long runs 163.0, 170.1, 164.6, 167.9;
+// 2.66 GB of short rows 481, 436, 431, 436; 3.4 GB Group ZeRO 637, 605, 595, 597;
+// (eighths, 2^8, 2^10) 9.2 GB of short rows 1480, 1475, 1472; 28 GB 4303, 4339,
+// 4290; 42 GB 6334, 6374, 6313; 70 GB 10660, 10703, 10678.  Runs of 2^4 were 8-13%
+// slower on the large ones.
+constexpr uint32_t kXcdRunLog2 = 8;
+constexpr uint32_t kXcdLongRunLog2 = 10;
+constexpr uint64_t kXcdLongRunMinChunks = 1ull << 19;
 constexpr uint64_t kMaxUnitsPerSeg = 1ull << 30;       // keeps unit math in 32 bits
 // Units per lane of a comparison's first pass.  Same allocations, calls of 4 / 2
 // / 1 units: 9.2 GB in short rows 1375 / 1338 / 1335 us, 28 GB 4004 / 3975 /
@@ -140,7 +150,7 @@ static_assert(2 * sizeof(Bases) + sizeof(SegHint) + 64 <= 4096, "kernel argument
 struct Tuning {
   std::atomic<uint32_t> blocks_per_cu{0};  // persistent grid: 0 = as many as can be resident
   std::atomic<uint32_t> nontemporal{1};
-  std::atomic<uint32_t> xcd_remap{1};      // 0, 1 (by plan size) or 2
+  std::atomic<uint32_t> xcd_remap{1};      // 0, or 1 and 2: runs of pieces per XCD
   std::atomic<uint32_t> run{4};            // persistent grid: round-robin runs of 4 x kUnroll chunks
   std::atomic<uint32_t> persistent{0};     // 0: one workgroup per piece of a chunk
   std::atomic<uint32_t> lanes{64};         // lanes per workgroup of one piece: 64, 128 or 256
@@ -729,21 +739,14 @@ __device__ __forceinline__ void warm_tables(const uint32_t *chunk_seg, const Dev
 // about 20% slower than 64 lanes of four); with the table, 1 KB pieces are
 // the fastest shape.
 //
-// xcd_share != 0: the first 8 * xcd_share workgroups are renumbered so that
-// each XCD (the hardware deals workgroups out to the 8 XCDs round-robin, so
-// workgroup w runs on XCD w % 8) works through one contiguous share of them,
-// in order: workgroup w takes piece (w % 8) * xcd_share + w / 8.  The
-// workgroups resident on one XCD then touch a window of the plan one eighth
-// as wide as when all eight XCDs share one window, so that XCD's L2 and
-// address-translation caches hold fewer pages at a time.  The rest (fewer
-// than 8) keep their own numbers.
+// xcd_end != 0: pieces are dealt out to the XCDs in runs; see xcd_order.
 template <bool kNT, bool kTable, int L, int U, bool kBuf>
 __global__ __launch_bounds__(L) void copy_plan_kernel(const DevSeg *__restrict__ segs, uint64_t n_chunks,
                                                       SegHint hint, Bases src, Bases dst,
                                                       const uint64_t *__restrict__ src_tab,
-                                                      const uint64_t *__restrict__ dst_tab, uint64_t xcd_share,
-                                                      const uint32_t *__restrict__ chunk_seg, uint32_t n_warm,
-                                                      uint32_t n_segs) {
+                                                      const uint64_t *__restrict__ dst_tab, uint64_t xcd_end,
+                                                      uint32_t xcd_log2, const uint32_t *__restrict__ chunk_seg,
+                                                      uint32_t n_warm, uint32_t n_segs) {
   constexpr uint32_t kPieces = kChunkUnits / (L * U);  // pieces per chunk: 1, 2 or 4
   static_assert(kPieces * L * U == kChunkUnits, "a piece divides a chunk");
   uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
@@ -752,7 +755,7 @@ __global__ __launch_bounds__(L) void copy_plan_kernel(const DevSeg *__restrict__
     return;
   }
   w -= n_warm;
-  if (w < xcd_share * 8) w = (w & 7) * xcd_share + (w >> 3);
+  w = xcd_order(w, xcd_end, xcd_log2);
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;
   uint32_t lo;
@@ -793,8 +796,8 @@ __global__ __launch_bounds__(L) void copy_plan_kernel(const DevSeg *__restrict__
 template <bool kNT, bool kTable, int L, int U, typename B>
 __global__ __launch_bounds__(L) void copy_pieces_kernel(const uint32_t *__restrict__ chunk_seg,
                                                         const DevSeg *__restrict__ segs, uint64_t n_chunks,
-                                                        uint64_t xcd_share, uint32_t gx, uint32_t n_warm,
-                                                        const uint64_t *__restrict__ src_tab,
+                                                        uint64_t xcd_end, uint32_t gx, uint32_t n_warm,
+                                                        uint32_t xcd_log2, const uint64_t *__restrict__ src_tab,
                                                         const uint64_t *__restrict__ dst_tab, B src, B dst,
                                                         uint32_t n_segs) {
   constexpr uint32_t kPieces = kChunkUnits / (L * U);  // pieces per chunk: 1, 2 or 4
@@ -805,7 +808,7 @@ __global__ __launch_bounds__(L) void copy_pieces_kernel(const uint32_t *__restri
     return;
   }
   w -= n_warm;
-  if (w < xcd_share * 8) w = (w & 7) * xcd_share + (w >> 3);
+  w = xcd_order(w, xcd_end, xcd_log2);
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;
   const DevSeg s = load_seg(segs + chunk_seg[c]);
@@ -1701,7 +1704,7 @@ __device__ __forceinline__ void differ_rows(const DevSeg &s, const char *sbase, 
 // chain of scalar loads (see copy_pieces_kernel): the first workgroups read the
 // tables, then one 64-lane workgroup per piece of U units a lane takes its
 // segment from the plan's chunk table, dispatched in order and, on large plans,
-// each XCD on its own eighth of the pieces.  Faster than the persistent grid on
+// XCDs in runs (xcd_order).  Faster than the persistent grid on
 // every full-size switch (2-4%, same allocations): a segment's rows or gathered
 // runs are spread over many workgroups in flight.  Bound by reading HBM.  Whole
 // calls before the pre-read, the preloaded arguments, two units a lane and the
@@ -1710,8 +1713,8 @@ __device__ __forceinline__ void differ_rows(const DevSeg &s, const char *sbase, 
 // 1567 and 1338, 28 GB 4016 and 3975, 44 GB 6437 and 6412.
 template <bool kTable, int U, typename B>
 __global__ __launch_bounds__(64) void differ_piece_kernel(
-    const uint32_t *__restrict__ chunk_seg, const DevSeg *__restrict__ segs, uint64_t n_chunks, uint64_t xcd_share,
-    uint32_t gx, uint32_t n_warm, const uint64_t *__restrict__ src_tab, const uint64_t *__restrict__ dst_tab, B src,
+    const uint32_t *__restrict__ chunk_seg, const DevSeg *__restrict__ segs, uint64_t n_chunks, uint64_t xcd_end,
+    uint32_t gx, uint32_t n_warm, uint32_t xcd_log2, const uint64_t *__restrict__ src_tab, const uint64_t *__restrict__ dst_tab, B src,
     B dst, uint32_t n_segs, DifferMarks marks) {
   constexpr uint32_t kPieces = kChunkUnits / (64 * U);
   uint64_t w = (uint64_t)blockIdx.y * gx + blockIdx.x;
@@ -1720,7 +1723,7 @@ __global__ __launch_bounds__(64) void differ_piece_kernel(
     return;
   }
   w -= n_warm;
-  if (w < xcd_share * 8) w = (w & 7) * xcd_share + (w >> 3);
+  w = xcd_order(w, xcd_end, xcd_log2);
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;
   const uint32_t lo = chunk_seg[c];
@@ -1955,6 +1958,20 @@ bool tight_grid(uint64_t n_wg, uint32_t lanes, dim3 *grid) {
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
+// How the pieces of `units` units are dealt out to the XCDs (xcd_order).
+struct XcdRuns {
+  uint64_t end;   // pieces dealt out in runs, the rest in the hardware's order
+  uint32_t log2;  // pieces per run
+};
+// For a plan of n_chunks chunks, cut into `per_chunk` (a power of two) pieces each.
+XcdRuns xcd_runs(uint64_t n_chunks, uint32_t per_chunk) {
+  if (!g_tuning.xcd_remap.load()) return XcdRuns{0, 0};
+  const uint64_t pieces = n_chunks * per_chunk;
+  uint32_t lg = n_chunks >= kXcdLongRunMinChunks ? kXcdLongRunLog2 : kXcdRunLog2;
+  for (; per_chunk > 1; per_chunk >>= 1) ++lg;
+  return XcdRuns{pieces >> (lg + 3) << (lg + 3), lg};
+}
+
 // Workgroups that read a plan's tables ahead of the pieces, a multiple of 8 so that the pieces keep their XCDs.
 uint32_t warm_groups(uint64_t n_chunks, uint64_t n_segs, uint32_t lanes) {
   const uint64_t units = n_chunks / 4 + n_segs * (sizeof(DevSeg) / sizeof(u32x4));
@@ -2058,21 +2075,19 @@ hipError_t differ_launch(const emrs_plan *plan, const CompareJob &job, const Dev
     const uint32_t n_warm = g_tuning.warm_tables.load() ? warm_groups(plan->n_chunks, nd, 64) : 0;
     dim3 grid;
     if (!tight_grid(n_warm + n_pieces, 64, &grid)) return hipErrorInvalidConfiguration;
-    const uint32_t remap = g_tuning.xcd_remap.load();
-    const bool by_xcd = remap == 2 || (remap == 1 && plan->n_chunks >= kXcdRemapMinChunks);
-    const uint64_t xcd_share = by_xcd ? n_pieces / 8 : 0;
+    const XcdRuns xcd = xcd_runs(plan->n_chunks, kChunkUnits / (64 * U));
     FewBases src{}, dst{};
     if (!job.rb.table)
       for (uint32_t i = 0; i < kFewBuffers; ++i) src.p[i] = job.rb.src.p[i], dst.p[i] = job.rb.dst.p[i];
     if (job.rb.table)
       hipLaunchKernelGGL((differ_piece_kernel<true, U, FewBases>), grid, dim3(64), 0, st, job.cseg, table,
-                         plan->n_chunks, xcd_share, grid.x, n_warm, tab, dtab, src, dst, nd, marks);
+                         plan->n_chunks, xcd.end, grid.x, n_warm, xcd.log2, tab, dtab, src, dst, nd, marks);
     else if (std::max(plan->stats.n_src_bufs, plan->stats.n_dst_bufs) <= kFewBuffers)
       hipLaunchKernelGGL((differ_piece_kernel<false, U, FewBases>), grid, dim3(64), 0, st, job.cseg, table,
-                         plan->n_chunks, xcd_share, grid.x, n_warm, tab, dtab, src, dst, nd, marks);
+                         plan->n_chunks, xcd.end, grid.x, n_warm, xcd.log2, tab, dtab, src, dst, nd, marks);
     else
       hipLaunchKernelGGL((differ_piece_kernel<false, U, Bases>), grid, dim3(64), 0, st, job.cseg, table,
-                         plan->n_chunks, xcd_share, grid.x, n_warm, tab, dtab, job.rb.src, job.rb.dst, nd, marks);
+                         plan->n_chunks, xcd.end, grid.x, n_warm, xcd.log2, tab, dtab, job.rb.src, job.rb.dst, nd, marks);
     return hipGetLastError();
   }
   // It could hold 8 workgroups per CU; 3-6 read at the plain read rate and 8 is up to
@@ -2409,39 +2424,37 @@ struct CopyLaunch {
 };
 
 template <bool kNT, bool kTable, int L, int U, bool kBuf>
-void launch_kernel(const CopyLaunch &c, dim3 grid, uint64_t xcd_share, uint32_t n_warm) {
+void launch_kernel(const CopyLaunch &c, dim3 grid, const XcdRuns &xcd, uint32_t n_warm) {
   if constexpr (!kBuf) {
     if (c.cseg) {
       if (c.n_bufs <= kFewBuffers || kTable) {
         FewBases src{}, dst{};
         for (uint32_t i = 0; i < kFewBuffers && !kTable; ++i) src.p[i] = c.rb->src.p[i], dst.p[i] = c.rb->dst.p[i];
         hipLaunchKernelGGL((copy_pieces_kernel<kNT, kTable, L, U, FewBases>), grid, dim3(L), 0, c.st, c.cseg, c.table,
-                           c.n_chunks, xcd_share, grid.x, n_warm, c.stab, c.dtab, src, dst, c.n_segs);
+                           c.n_chunks, xcd.end, grid.x, n_warm, xcd.log2, c.stab, c.dtab, src, dst, c.n_segs);
       } else if constexpr (!kTable) {
         hipLaunchKernelGGL((copy_pieces_kernel<kNT, false, L, U, Bases>), grid, dim3(L), 0, c.st, c.cseg, c.table,
-                           c.n_chunks, xcd_share, grid.x, n_warm, c.stab, c.dtab, c.rb->src, c.rb->dst, c.n_segs);
+                           c.n_chunks, xcd.end, grid.x, n_warm, xcd.log2, c.stab, c.dtab, c.rb->src, c.rb->dst, c.n_segs);
       }
       return;
     }
   }
   hipLaunchKernelGGL((copy_plan_kernel<kNT, kTable, L, U, kBuf>), grid, dim3(L), 0, c.st, c.table, c.n_chunks, *c.hint,
-                     c.rb->src, c.rb->dst, c.stab, c.dtab, xcd_share, c.cseg, n_warm, c.n_segs);
+                     c.rb->src, c.rb->dst, c.stab, c.dtab, xcd.end, xcd.log2, c.cseg, n_warm, c.n_segs);
 }
 
 template <int L, int U, bool kBuf>
 int launch_chunks(const CopyLaunch &c) {
   const uint64_t n_pieces = c.n_chunks * (kChunkUnits / (L * U));
-  const uint32_t remap = g_tuning.xcd_remap.load();
-  const bool by_xcd = remap == 2 || (remap == 1 && c.n_chunks >= kXcdRemapMinChunks);
-  const uint64_t xcd_share = by_xcd ? n_pieces / 8 : 0;
+  const XcdRuns xcd = xcd_runs(c.n_chunks, kChunkUnits / (L * U));
   const uint64_t n_warm = c.cseg && c.warm ? warm_groups(c.n_chunks, c.n_segs, L) : 0;
   dim3 grid;
   if (!tight_grid(n_warm + n_pieces, L, &grid))
     return fail(EMRS_ERR_INVALID_ARGUMENT, "plan has too many chunks for one launch");
-  if (c.nt && c.rb->table) launch_kernel<true, true, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
-  else if (c.nt) launch_kernel<true, false, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
-  else if (c.rb->table) launch_kernel<false, true, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
-  else launch_kernel<false, false, L, U, kBuf>(c, grid, xcd_share, (uint32_t)n_warm);
+  if (c.nt && c.rb->table) launch_kernel<true, true, L, U, kBuf>(c, grid, xcd, (uint32_t)n_warm);
+  else if (c.nt) launch_kernel<true, false, L, U, kBuf>(c, grid, xcd, (uint32_t)n_warm);
+  else if (c.rb->table) launch_kernel<false, true, L, U, kBuf>(c, grid, xcd, (uint32_t)n_warm);
+  else launch_kernel<false, false, L, U, kBuf>(c, grid, xcd, (uint32_t)n_warm);
   return EMRS_OK;
 }
 

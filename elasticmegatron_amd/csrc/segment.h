@@ -147,6 +147,18 @@ EMRS_HD inline RowUnit row_unit(const DevSeg &s, const char *dbase, uint32_t u, 
   return r;
 }
 
+// Piece of workgroup `w`.  The hardware deals workgroups out to the 8 XCDs
+// round-robin (workgroup w runs on XCD w % 8); the first `end` of them (whole
+// blocks of 8 << lg) are renumbered so that each XCD works through a run of
+// 1 << lg consecutive pieces of every block, in order.  The pieces resident on
+// one XCD then lie together, so that its L2 holds whole what two neighbours
+// share, and its translation caches fewer pages.
+EMRS_HD inline uint64_t xcd_order(uint64_t w, uint64_t end, uint32_t lg) {
+  if (w >= end) return w;
+  const uint64_t i = w & ((8ull << lg) - 1);
+  return w - i + ((i & 7) << lg) + (i >> 3);
+}
+
 }  // namespace emrs_internal
 
 #endif  // EMRS_SEGMENT_H

@@ -381,7 +381,8 @@ class TransferManager:
         # tensors, and this check runs before every launch.  The pointers and sizes are read on
         # every call; the layout and device checks are skipped when both equal those of the last
         # call that passed them (the same tensors again: same storage, offset and size).
-        # That no tensor is None shows in the first pass (with a pass of its own and numpy's pointer arrays, 900 small tensors took 112 us a call, now 94).
+        # That no tensor is None shows in the first pass (with a pass of its own and numpy's pointer
+        # arrays, 900 small tensors took 112 us a call, now 94).
         try:
             ptrs = [t.data_ptr() for t in ts]
         except Exception:

@@ -283,11 +283,12 @@ typedef struct emrs_tuning {
   uint32_t blocks_per_cu; /* workgroups per CU in the persistent grid (0..64);
                              0 (default): as many as can be resident at once */
   uint32_t nontemporal;   /* 1: streaming (non-temporal) loads and stores (default 1) */
-  uint32_t xcd_remap;     /* 0, 1 (default) or 2.  Nonzero: each XCD works through one contiguous
-                             eighth of the chunks (workgroup b runs on XCD b % 8); the persistent
-                             grid does so for 1 and 2, one workgroup per piece for 2 and, with 1,
-                             for plans of at least 2^19 chunks.  0: workgroup b takes piece b (one
-                             workgroup per piece) or the b-th run (persistent) */
+  uint32_t xcd_remap;     /* 0, 1 (default) or 2.  Nonzero: each XCD works through contiguous parts of the
+                             plan (workgroup b runs on XCD b % 8): with one workgroup per piece, runs of
+                             2^8 chunks, of 2^10 in plans of at least 2^19 chunks, dealt out in turn; in
+                             the persistent grid, one eighth of the chunks.  1 and 2 are the same.
+                             0: workgroup b takes piece b (one workgroup per piece) or the b-th run
+                             (persistent) */
   uint32_t run;           /* persistent grid, 0: each workgroup copies one contiguous run of
                              chunks; N in [1, 2^20]: chunks are dealt out round-robin in runs of
                              8N, capped at a quarter of a workgroup's share (default 4) */
