@@ -89,6 +89,12 @@ constexpr int kUnroll = EMRS_COPY_UNROLL;
 constexpr uint32_t kChunkUnits = kThreads;  // units per work chunk: one per lane
 constexpr uint32_t kStepUnits = kThreads * kUnroll;  // units per step of a persistent workgroup
 constexpr uint64_t kMaxGridY = 65535;                     // rows of a one-workgroup-per-chunk grid
+// Row units per lane and step in copy_plan_persistent_kernel and differ_plan_kernel.  A kernel's
+// registers are those of its largest path, whatever a plan holds: with kUnroll row units in flight they
+// took 312-316 vector registers and 80 bytes of scratch, and 91, so that one and five waves fitted on a
+// SIMD; with two, 83 (five waves) and 50 (eight).  Persistent grid, us with kUnroll and with two: 1.0 GB
+// 293 and 206, 28 GB 6299 and 5451, 9.2 GB in short rows 3675 and 2050.
+constexpr int kRowStep = 2;
 // Chunks in a run of one XCD (see xcd_order): 2^8 (1 MB of 16-byte units), and
 // 2^10 in plans of at least 2^19 chunks.  Before, such plans gave each XCD an
 // eighth of all their chunks, and smaller ones kept the hardware's order, which
@@ -390,7 +396,9 @@ __device__ __forceinline__ void copy_chunk_run(const DevSeg *__restrict__ segs, 
     char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
     const uint32_t ops = s.ops(), ul = s.unit_log2();
     if (ul == kRowUnits) {
-      dispatch_rows<kNT, kThreads, kUnroll>(s, sb, db, ab, u0, u_end);
+#pragma unroll 1
+      for (uint32_t u = u0; u < u_end; u += kThreads * kRowStep)
+        dispatch_rows<kNT, kThreads, kRowStep>(s, sb, db, ab, u, u_end);
       continue;
     }
     if (ops & 4) {  // duplicate to aux, with or without zero fill
@@ -1794,7 +1802,11 @@ __global__ __launch_bounds__(kThreads) void differ_plan_kernel(
       const char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
       const char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
       switch (s.unit_log2()) {
-        case kRowUnits: differ_rows<kThreads, kUnroll>(s, sb, db, ab, u0, u_end, dm, dx); break;
+        case kRowUnits:
+#pragma unroll 1
+          for (uint32_t u = u0; u < u_end; u += kThreads * kRowStep)
+            differ_rows<kThreads, kRowStep>(s, sb, db, ab, u, u_end, dm, dx);
+          break;
         case 4: differ_chunk<u32x4>(s, sb, db, ab, u0, u_end, dm, dx); break;
         case 3: differ_chunk<uint64_t>(s, sb, db, ab, u0, u_end, dm, dx); break;
         case 2: differ_chunk<uint32_t>(s, sb, db, ab, u0, u_end, dm, dx); break;
