@@ -155,8 +155,8 @@ def parse():
     ap.add_argument("--blocks-per-cu", type=int, default=0, help="persistent grid; 0: as many as can be resident")
     ap.add_argument("--nontemporal", type=int, default=1)
     ap.add_argument("--xcd-remap", type=int, default=1, choices=(0, 1, 2),
-                    help="each XCD takes one contiguous eighth of the chunks: 1 in the persistent grid and for "
-                         "plans of at least 2^19 chunks, 2 always, 0 never")
+                    help="how pieces are dealt out to the XCDs: 0 in the hardware's order, 1 in runs of 2^8 chunks "
+                         "(2^10 in plans of at least 2^19), 2 one eighth each (persistent grid: 1 and 2 an eighth each)")
     ap.add_argument("--run", type=int, default=4,
                     help="persistent grid; 0: contiguous chunk run per workgroup; N: round-robin runs of 8N chunks")
     ap.add_argument("--megatron-buffers", action="store_true",

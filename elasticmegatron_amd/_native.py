@@ -178,11 +178,11 @@ def set_tuning(blocks_per_cu: int = 0, nontemporal: bool = True, xcd_remap: int 
     (0: 64) with ``units`` 16-byte units each (0: a whole chunk of 256 units per workgroup) per piece
     of a chunk, each finding its segment in the plan's chunk table (``chunk_index``; False: by a
     bounded binary search); ``persistent=True`` selects a persistent grid, which ``blocks_per_cu``
-    and ``run`` shape.  ``xcd_remap`` (1, or 2 alike) has each of the 8 XCDs work through runs of
-    consecutive chunks (the persistent grid: through one eighth of them); 0 (or False) keeps the
-    hardware's order.  ``warm_tables``: with the chunk table, the first workgroups of each copy launch
-    read it and the segment descriptors, so that a launch after unrelated work starts from cached
-    tables."""
+    and ``run`` shape.  ``xcd_remap`` 1 (or True) has each of the 8 XCDs work through runs of
+    consecutive chunks, 2 through one eighth of the pieces (the persistent grid: an eighth of the chunks
+    for both); 0 (or False) keeps the hardware's order.  ``warm_tables``: with the chunk table, the first
+    workgroups of each copy launch read it and the segment descriptors, so that a launch after unrelated
+    work starts from cached tables."""
     t = Tuning(blocks_per_cu, 1 if nontemporal else 0, int(xcd_remap), run, 1 if persistent else 0, lanes,
                units, 1 if buffer_ops else 0, 1 if chunk_index else 0, 1 if warm_tables else 0)
     _check(load().emrs_set_tuning(ctypes.byref(t)), "emrs_set_tuning")

@@ -95,21 +95,6 @@ constexpr uint64_t kMaxGridY = 65535;                     // rows of a one-workg
 // SIMD; with two, 83 (five waves) and 50 (eight).  Persistent grid, us with kUnroll and with two: 1.0 GB
 // 293 and 206, 28 GB 6299 and 5451, 9.2 GB in short rows 3675 and 2050.
 constexpr int kRowStep = 2;
-// Chunks in a run of one XCD (see xcd_order): 2^8 (1 MB of 16-byte units), and
-// 2^10 in plans of at least 2^19 chunks.  Before, such plans gave each XCD an
-// eighth of all their chunks, and smaller ones kept the hardware's order, which
-// splits neighbouring kilobytes over XCDs: lines and pages at their ends are
-// then fetched by two of them, the more the less aligned the rows are.  us (hardware
-// order, eighths, runs of 2^8, of 2^10), one process, same allocations: 0.1 GB
-// 30.7, 27.0, 29.1, 28.1; 0.55 GB of short rows 107.7, 99.9, 99.4, 99.2; 0.93 GB
-// 164.6, 155.8, 155.4, 155.8; 1.02 GB of long runs 163.0, 170.1, 164.6, 167.9;
-// 2.66 GB of short rows 481, 436, 431, 436; 3.4 GB Group ZeRO 637, 605, 595, 597;
-// (eighths, 2^8, 2^10) 9.2 GB of short rows 1480, 1475, 1472; 28 GB 4303, 4339,
-// 4290; 42 GB 6334, 6374, 6313; 70 GB 10660, 10703, 10678.  Runs of 2^4 were 8-13%
-// slower on the large ones.
-constexpr uint32_t kXcdRunLog2 = 8;
-constexpr uint32_t kXcdLongRunLog2 = 10;
-constexpr uint64_t kXcdLongRunMinChunks = 1ull << 19;
 constexpr uint64_t kMaxUnitsPerSeg = 1ull << 30;       // keeps unit math in 32 bits
 // Units per lane of a comparison's first pass.  Same allocations, calls of 4 / 2
 // / 1 units: 9.2 GB in short rows 1375 / 1338 / 1335 us, 28 GB 4004 / 3975 /
@@ -156,7 +141,7 @@ static_assert(2 * sizeof(Bases) + sizeof(SegHint) + 64 <= 4096, "kernel argument
 struct Tuning {
   std::atomic<uint32_t> blocks_per_cu{0};  // persistent grid: 0 = as many as can be resident
   std::atomic<uint32_t> nontemporal{1};
-  std::atomic<uint32_t> xcd_remap{1};      // 0, or 1 and 2: runs of pieces per XCD
+  std::atomic<uint32_t> xcd_remap{1};      // 0: hardware's order; 1: runs of pieces per XCD; 2: eighths
   std::atomic<uint32_t> run{4};            // persistent grid: round-robin runs of 4 x kUnroll chunks
   std::atomic<uint32_t> persistent{0};     // 0: one workgroup per piece of a chunk
   std::atomic<uint32_t> lanes{64};         // lanes per workgroup of one piece: 64, 128 or 256
@@ -1970,20 +1955,6 @@ bool tight_grid(uint64_t n_wg, uint32_t lanes, dim3 *grid) {
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-// How the pieces of `units` units are dealt out to the XCDs (xcd_order).
-struct XcdRuns {
-  uint64_t end;   // pieces dealt out in runs, the rest in the hardware's order
-  uint32_t log2;  // pieces per run
-};
-// For a plan of n_chunks chunks, cut into `per_chunk` (a power of two) pieces each.
-XcdRuns xcd_runs(uint64_t n_chunks, uint32_t per_chunk) {
-  if (!g_tuning.xcd_remap.load()) return XcdRuns{0, 0};
-  const uint64_t pieces = n_chunks * per_chunk;
-  uint32_t lg = n_chunks >= kXcdLongRunMinChunks ? kXcdLongRunLog2 : kXcdRunLog2;
-  for (; per_chunk > 1; per_chunk >>= 1) ++lg;
-  return XcdRuns{pieces >> (lg + 3) << (lg + 3), lg};
-}
-
 // Workgroups that read a plan's tables ahead of the pieces, a multiple of 8 so that the pieces keep their XCDs.
 uint32_t warm_groups(uint64_t n_chunks, uint64_t n_segs, uint32_t lanes) {
   const uint64_t units = n_chunks / 4 + n_segs * (sizeof(DevSeg) / sizeof(u32x4));
@@ -2087,7 +2058,7 @@ hipError_t differ_launch(const emrs_plan *plan, const CompareJob &job, const Dev
     const uint32_t n_warm = g_tuning.warm_tables.load() ? warm_groups(plan->n_chunks, nd, 64) : 0;
     dim3 grid;
     if (!tight_grid(n_warm + n_pieces, 64, &grid)) return hipErrorInvalidConfiguration;
-    const XcdRuns xcd = xcd_runs(plan->n_chunks, kChunkUnits / (64 * U));
+    const XcdRuns xcd = xcd_runs(g_tuning.xcd_remap.load(), plan->n_chunks, kChunkUnits / (64 * U));
     FewBases src{}, dst{};
     if (!job.rb.table)
       for (uint32_t i = 0; i < kFewBuffers; ++i) src.p[i] = job.rb.src.p[i], dst.p[i] = job.rb.dst.p[i];
@@ -2458,7 +2429,7 @@ void launch_kernel(const CopyLaunch &c, dim3 grid, const XcdRuns &xcd, uint32_t 
 template <int L, int U, bool kBuf>
 int launch_chunks(const CopyLaunch &c) {
   const uint64_t n_pieces = c.n_chunks * (kChunkUnits / (L * U));
-  const XcdRuns xcd = xcd_runs(c.n_chunks, kChunkUnits / (L * U));
+  const XcdRuns xcd = xcd_runs(g_tuning.xcd_remap.load(), c.n_chunks, kChunkUnits / (L * U));
   const uint64_t n_warm = c.cseg && c.warm ? warm_groups(c.n_chunks, c.n_segs, L) : 0;
   dim3 grid;
   if (!tight_grid(n_warm + n_pieces, L, &grid))

@@ -284,11 +284,11 @@ typedef struct emrs_tuning {
                              0 (default): as many as can be resident at once */
   uint32_t nontemporal;   /* 1: streaming (non-temporal) loads and stores (default 1) */
   uint32_t xcd_remap;     /* 0, 1 (default) or 2.  Nonzero: each XCD works through contiguous parts of the
-                             plan (workgroup b runs on XCD b % 8): with one workgroup per piece, runs of
-                             2^8 chunks, of 2^10 in plans of at least 2^19 chunks, dealt out in turn; in
-                             the persistent grid, one eighth of the chunks.  1 and 2 are the same.
-                             0: workgroup b takes piece b (one workgroup per piece) or the b-th run
-                             (persistent) */
+                             plan (workgroup b runs on XCD b % 8).  One workgroup per piece, 1: runs of
+                             2^8 chunks, of 2^10 in plans of at least 2^19 chunks, dealt out in turn; 2:
+                             one eighth of the pieces.  Persistent grid, 1 and 2: one eighth of the
+                             chunks.  0: workgroup b takes piece b (one workgroup per piece) or the b-th
+                             run (persistent) */
   uint32_t run;           /* persistent grid, 0: each workgroup copies one contiguous run of
                              chunks; N in [1, 2^20]: chunks are dealt out round-robin in runs of
                              8N, capped at a quarter of a workgroup's share (default 4) */
