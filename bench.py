@@ -478,13 +478,15 @@ def main():
 def committed_traffic(workload: str, bf16_source, algorithmic_bytes: int):
     """HBM bytes per launch from the committed PMC summary of ``workload`` (profiles/), or None when
     there is none for this bf16 source (None: fp32-only Group-ZeRO plans) or it was measured on a
-    plan with other algorithmic bytes."""
+    plan with other algorithmic bytes, with another kernel or in another launch shape."""
     tf = os.path.join(ROOT, "profiles", f"{workload}.traffic.json")
     if not os.path.exists(tf):
         return None
     with open(tf) as f:
         rec = json.load(f)
     if rec.get("bf16_source", "cast") != bf16_source or rec.get("algorithmic_bytes_per_launch") != algorithmic_bytes:
+        return None
+    if rec.get("kernel") != copy_kernel() or rec.get("launch") != launch_shape():
         return None
     return rec.get("hbm_bytes_per_launch")
 
@@ -1389,6 +1391,16 @@ def launch_shape():
             "piece_bytes": 16 * t.lanes * t.units, "chunk_index": t.chunk_index, "warm_tables": t.warm_tables,
             "xcd_remap": t.xcd_remap,
             "buffer_ops": t.buffer_ops, "nontemporal": t.nontemporal}
+
+
+def copy_kernel():
+    """The kernel that a switch launches in the launch shape in effect."""
+    from elasticmegatron_amd import _native
+
+    t = _native.get_tuning()
+    if t.persistent:
+        return "copy_plan_persistent_kernel"
+    return "copy_pieces_kernel" if t.chunk_index and not t.buffer_ops else "copy_plan_kernel"
 
 
 def alternate_rounds(runs, stream, rounds=3, reps=5):

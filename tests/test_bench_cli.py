@@ -102,6 +102,42 @@ def test_committed_traffic_describes_the_current_plan(traffic_file):
     assert bench.committed_traffic(name, "cast" if backup is None else None, plan.traffic_bytes + 1) is None
 
 
+@pytest.mark.parametrize("change", [dict(kernel="copy_plan_kernel"), dict(kernel=None), dict(launch=None),
+                                    dict(tuning=dict(xcd_remap=2)), dict(tuning=dict(units=2)),
+                                    dict(tuning=dict(chunk_index=False)), dict(tuning=dict(persistent=True))])
+def test_committed_traffic_of_another_kernel_or_launch_shape_is_not_quoted(tmp_path, monkeypatch, change):
+    """Counters of an earlier kernel, or of another launch shape, are not those of the launch at hand."""
+    from elasticmegatron_amd import _native
+
+    name = bench.HEADLINE
+    with open(os.path.join(ROOT, "profiles", name + ".traffic.json")) as f:
+        rec = json.load(f)
+    n = rec["algorithmic_bytes_per_launch"]
+    assert bench.committed_traffic(name, "cast", n) == rec["hbm_bytes_per_launch"]
+    rec.update({k: v for k, v in change.items() if k != "tuning"})
+    (tmp_path / "profiles").mkdir()
+    (tmp_path / "profiles" / (name + ".traffic.json")).write_text(json.dumps(rec))
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    try:
+        _native.set_tuning(**change.get("tuning", {}))
+        assert bench.committed_traffic(name, "cast", n) is None
+    finally:
+        _native.set_tuning()
+
+
+def test_the_kernel_named_is_one_of_the_library():
+    from elasticmegatron_amd import _native, build
+
+    with open(build.LIB, "rb") as f:
+        lib = f.read()
+    try:
+        for tuning in ({}, dict(buffer_ops=True), dict(chunk_index=False), dict(persistent=True)):
+            _native.set_tuning(**tuning)
+            assert bench.copy_kernel().encode() in lib, tuning
+    finally:
+        _native.set_tuning()
+
+
 @pytest.mark.parametrize("src,dst", [(ParallelStrategy(8, 2, 1), ParallelStrategy(8, 1, 1)),
                                      (ParallelStrategy(4, 1, 1),
                                       ParallelStrategy(8, 1, 1, num_distributed_optimizer_instances=2))])
