@@ -3,7 +3,8 @@
 Lengths around a workgroup's units, a chunk and several chunks; every element width and second
 destination; one planted element at the ends and inside, of the destination or of the second one.
 Counts are whole numbers: they must be exact.  After each find the plan compares clean again, so no
-mark outlives its call.
+mark outlives its call.  The allocation-free entry point also runs on a plan that has never run and
+so has no chunk table: its first pass is then the persistent one, without workgroups per piece.
 """
 
 import numpy as np
@@ -18,9 +19,10 @@ pytestmark = pytest.mark.gpu
 CAST, DUP = 1, 4
 
 
-@pytest.mark.parametrize("no_alloc", [False, True], ids=["compare", "compare_static"])
+@pytest.mark.parametrize("no_alloc,table", [(False, True), (True, True), (True, False)],
+                         ids=["compare", "compare_static", "compare_static_without_chunk_table"])
 @pytest.mark.parametrize("elem,flags", [(4, 0), (4, CAST), (4, DUP), (2, 0), (2, DUP), (1, 0), (8, DUP)])
-def test_one_element(gpu_device, elem, flags, no_alloc):
+def test_one_element(gpu_device, elem, flags, no_alloc, table):
     lens = [1, 3, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 4097, 9000]
     segs, off = [], 0
     for k, n in enumerate(lens):   # every other segment on 16 bytes, the rest an element off where they fall
@@ -38,13 +40,15 @@ def test_one_element(gpu_device, elem, flags, no_alloc):
     st = torch.cuda.current_stream(gpu_device).cuda_stream
     sp, dp = [src.data_ptr()], [dst.data_ptr(), aux.data_ptr()]
     plan.execute(sp, dp, st)
+    if not table:
+        plan = _native.Plan(t, [nbytes], [nbytes, nbytes])
     m = len(lens)
     groups, aux_groups = np.arange(m, dtype=np.uint32), np.arange(m, 2 * m, dtype=np.uint32)
 
     def mismatches():
         return plan.compare(sp, dp, groups, aux_groups, 2 * m, st, no_alloc=no_alloc)["mismatches"].astype(int)
 
-    print(f"case one element: {elem} bytes, flags {flags}, no_alloc {no_alloc}", flush=True)
+    print(f"case one element: {elem} bytes, flags {flags}, no_alloc {no_alloc}, chunk table {table}", flush=True)
     assert not mismatches().any()
     for k, n in enumerate(lens):
         for second in ([False, True] if flags else [False]):

@@ -107,10 +107,13 @@ def test_row_units_copy_and_compare(gpu_device, eb, tuning):
     assert not dst[:16].any() and not aux[:16].any()
 
     # Every element counted once; damage to the first, second, middle and last element of rows is found.
+    # The allocation-free entry point runs on a second plan too, one that has never run and so has no
+    # chunk table: its first pass is then the persistent one.
     n = len(t)
     groups = np.arange(n, dtype=np.uint32)
-    for no_alloc in (False, True):   # without a chunk table of its own, the second entry point may run another first pass
-        got = plan.compare(*bases, groups, groups + n, 2 * n, st, no_alloc=no_alloc)
+    fresh = _native.Plan(t, [ns], [nd, na])
+    for p, no_alloc in ((fresh, True), (plan, False), (plan, True)):
+        got = p.compare(*bases, groups, groups + n, 2 * n, st, no_alloc=no_alloc)
         assert not got["mismatches"].any()
         assert np.array_equal(got["elements"][:n], t["len"] * t["rows"])
     d, hits = dst[16:].view({2: torch.int16, 4: torch.int32, 8: torch.int64}[eb]), np.zeros(n, dtype=np.uint64)
@@ -120,6 +123,14 @@ def test_row_units_copy_and_compare(gpu_device, eb, tuning):
         for c in cols:
             d[int(t[i]["dst_off"]) + r * int(t[i]["dst_stride"]) + c] ^= 1
         hits[i] = len(cols)
-    for no_alloc in (False, True):
-        got = plan.compare(*bases, groups, groups + n, 2 * n, st, no_alloc=no_alloc)
-        assert np.array_equal(got["mismatches"][:n], hits) and not got["mismatches"][n:].any()
+    aux_hits = np.zeros(n, dtype=np.uint64)   # the last element of the second destination's last row
+    for i in range(1, n, 3):
+        s, fl = t[i], int(t[i]["flags"])
+        if fl & 5:
+            at = int(s["aux_off"]) + (int(s["rows"]) - 1) * int(s["aux_stride"]) + int(s["len"]) - 1
+            aux[16 + at * (2 if fl & 1 else eb)] ^= 1
+            aux_hits[i] = 1
+    assert aux_hits.any()
+    for p, no_alloc in ((fresh, True), (plan, False), (plan, True)):
+        got = p.compare(*bases, groups, groups + n, 2 * n, st, no_alloc=no_alloc)
+        assert np.array_equal(got["mismatches"][:n], hits) and np.array_equal(got["mismatches"][n:], aux_hits)
