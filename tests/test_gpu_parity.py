@@ -288,7 +288,7 @@ def test_bf16_cast_rounding_special_values(gpu_device):
     aux = torch.zeros(n, dtype=torch.int16, device=gpu_device)
     t = np.zeros(2, dtype=SEGMENT_DTYPE)
     t[0] = (0, 0, 4, 1, 0, 0, n // 2, 1, 0, 0, 1, 0, 0, 0)           # vector path
-    t[1] = (0, 0, 4, 1, n // 2, n // 2, n // 2 - 1, 1, 0, 0, 1, 0, n // 2 + 1, 0)  # element path
+    t[1] = (0, 0, 4, 1, n // 2, n // 2, n // 2 - 1, 1, 0, 0, 1, 0, n // 2 + 1, 0)  # row units
     plan = _native.Plan(t, [n * 4], [n * 4, n * 2])
     assert plan.stats().scalar_bytes > 0 and plan.stats().vector_bytes > 0
     plan.execute([src.data_ptr()], [dst.data_ptr(), aux.data_ptr()], torch.cuda.current_stream().cuda_stream)
@@ -303,6 +303,39 @@ def test_bf16_cast_rounding_special_values(gpu_device):
     torch_bf16 = torch.from_numpy(host.view(np.float32)).to(torch.bfloat16).view(torch.int16).numpy().view(np.uint16)
     assert np.array_equal(want[:n // 2][finite[:n // 2]], torch_bf16[:n // 2][finite[:n // 2]])
     assert (want[~np.concatenate([finite[:n // 2], [True], finite[n // 2:n - 1]])] == 0x7FC0).all()
+
+
+@pytest.mark.parametrize("tuning", [{}, dict(buffer_ops=True), dict(persistent=True)])
+def test_bf16_cast_special_values_in_short_runs_and_rows(gpu_device, tuning):
+    """The cast of single elements: runs of 1 to 3, and rows of 3, which no 16-byte unit holds."""
+    vals = np.array([0x3F800000, 0x3F808000, 0x3F818000, 0x3F80FFFF, 0x7F7FFFFF, 0x7F800000, 0xFF800000,
+                     0x7FC00001, 0xFFFFFFFF, 0x80000000, 0x00000001, 0x807FFFFF, 0x3F7F7FFF, 0x3F7F8000,
+                     0x477FE000, 0xC2F6E979, 0x7F800001, 0xFF7F8000, 0x00008000], dtype=np.uint32)
+    host = np.tile(vals, 12)   # 228 values: 38 times runs of 1, 2 and 3, and 76 rows of 3
+    runs = [(6 * k + o, n) for k in range(38) for o, n in ((0, 1), (1, 2), (3, 3))]
+    t = np.zeros(len(runs) + 1, dtype=SEGMENT_DTYPE)
+    t[:-1] = [(0, 0, 4, 1, o, o, n, 1, 0, 0, 1, 0, o, 0) for o, n in runs]
+    t[-1] = (0, 0, 4, 1, 0, 300, 3, 76, 3, 4, 1, 0, 301, 5)
+    n_dst, n_aux = 300 + 76 * 4, 301 + 76 * 5
+    plan = _native.Plan(t, [host.nbytes], [n_dst * 4, n_aux * 2], check_disjoint=True)
+    assert plan.stats().vector_bytes == 0 and plan.stats().n_chunks == plan.stats().n_device_segments
+    src = torch.from_numpy(host.view(np.int32)).to(gpu_device)
+    dst = torch.zeros(n_dst, dtype=torch.int32, device=gpu_device)
+    aux = torch.zeros(n_aux, dtype=torch.int16, device=gpu_device)
+    print(f"case short casts, tuning {tuning}", flush=True)
+    try:
+        _native.set_tuning(**tuning)
+        plan.execute([src.data_ptr()], [dst.data_ptr(), aux.data_ptr()], torch.cuda.current_stream().cuda_stream)
+    finally:
+        _native.set_tuning()
+    torch.cuda.synchronize()
+    want, want_aux = np.zeros(n_dst, dtype=np.uint32), np.zeros(n_aux, dtype=np.uint16)
+    want[:228], want_aux[:228] = host, bf16_rne_bits(host)
+    for r in range(76):
+        want[300 + 4 * r:303 + 4 * r] = host[3 * r:3 * r + 3]
+        want_aux[301 + 5 * r:304 + 5 * r] = bf16_rne_bits(host[3 * r:3 * r + 3])
+    assert np.array_equal(dst.cpu().numpy().view(np.uint32), want)
+    assert np.array_equal(aux.cpu().numpy().view(np.uint16), want_aux)
 
 
 @pytest.mark.parametrize("tuning", [{}, dict(chunk_index=False), dict(units=4), dict(persistent=True)])

@@ -122,10 +122,12 @@ def test_too_many_buffers():
 
 
 def test_plan_stats_classify_alignment():
+    """The byte counts say how segments lie to 16 bytes; what moves them, the next test reads off the
+    device segments and chunks that the builder made."""
     z = (0, 0, 0, 0)
     rows = [
         (0, 0, 4, 0, 0, 0, 64, 1, 0, 0) + z,      # vector: 256 bytes
-        (0, 0, 4, 0, 1, 1, 12, 1, 0, 0) + z,      # co-aligned, 4 B off: 3 head + 8 body + 1 tail elements
+        (0, 0, 4, 0, 1, 1, 12, 1, 0, 0) + z,      # co-aligned, 4 B off: 8 of 12 elements fill 16-byte units
         (0, 0, 4, 0, 1, 2, 8, 1, 0, 0) + z,       # not co-aligned: scalar
         (0, 0, 2, 0, 0, 0, 8, 4, 16, 8) + z,      # strided bf16 rows of 16 bytes: vector
         (0, 0, 2, 0, 0, 64, 3, 4, 8, 5) + z,      # strided, odd: scalar
@@ -140,6 +142,43 @@ def test_plan_stats_classify_alignment():
     assert st.vector_bytes == 256 + 32 + 64 + 128
     assert st.scalar_bytes == 16 + 32 + 24 + 128
     assert st.n_segments == 7
+
+
+# One segment each: elem_bytes, flags, src_off, dst_off, len, rows, src_stride, dst_stride, aux_off,
+# aux_stride; and the device segments and chunks of 256 units that its route makes.
+ROUTES = {
+    # 16-byte units: 10000 / 4 of them.
+    "aligned": ((4, 0, 0, 0, 10000, 1, 0, 0, 0, 0), 1, 10),
+    "aligned rows": ((2, 0, 0, 8, 40, 100, 48, 56, 0, 0), 1, 2),
+    "aligned cast": ((4, 1, 0, 0, 10000, 1, 0, 0, 4, 0), 1, 10),
+    # Row units: those of a row that starts anywhere, (len + 31 + 3) / 4 of fp32.
+    "one element off, together": ((4, 0, 1, 1, 10000, 1, 0, 0, 0, 0), 1, 10),
+    "one element off": ((4, 0, 1, 2, 10000, 1, 0, 0, 0, 0), 1, 10),
+    "bf16 one element off": ((2, 0, 1, 2, 10000, 1, 0, 0, 0, 0), 1, 5),
+    "8 bytes one element off": ((8, 0, 0, 1, 1000, 1, 0, 0, 0, 0), 1, 2),
+    "no whole units": ((4, 0, 0, 0, 10001, 1, 0, 0, 0, 0), 1, 10),
+    "image off": ((4, 1, 0, 0, 10000, 1, 0, 0, 1, 0), 1, 10),
+    "duplicate off": ((4, 4, 0, 0, 10000, 1, 0, 0, 1, 0), 1, 10),
+    "zeros off": ((4, 2, 0, 1, 10000, 1, 0, 0, 0, 0), 1, 10),
+    "pitched rows": ((4, 0, 0, 0, 40, 100, 41, 43, 0, 0), 1, 5),          # 11 units a row, on 16 bytes
+    "pitched long rows": ((4, 0, 0, 0, 128, 100, 129, 130, 0, 0), 1, 16),  # 40 units a row, on lines
+    # Elements: rows of under 16 bytes, and bytes.
+    "short rows": ((4, 0, 0, 0, 3, 100, 5, 4, 0, 0), 1, 2),
+    "short run": ((4, 1, 5, 9, 3, 1, 0, 0, 1, 0), 1, 1),
+    "bytes": ((1, 0, 1, 2, 10000, 1, 0, 0, 0, 0), 1, 40),
+    "bytes, together": ((1, 0, 1, 1, 10000, 1, 0, 0, 0, 0), 3, 5),        # 15 elements, 624 units, 1 element
+    "byte rows": ((1, 0, 0, 0, 100, 100, 101, 103, 0, 0), 1, 40),
+}
+
+
+@pytest.mark.parametrize("name", ROUTES)
+def test_route_of_a_segment(name):
+    """Which unit moves a segment shows in the number of chunks: a unit of its elements, or of 16 bytes."""
+    (eb, fl, so, do, n, rows, ss, ds, ao, as_), segments, chunks = ROUTES[name]
+    t = np.zeros(1, dtype=SEGMENT_DTYPE)
+    t[0] = (0, 0, eb, fl, so, do, n, rows, ss, ds, 1 if fl & 5 else 0, 0, ao, as_)
+    st = _native.Plan(t, [1 << 20], [1 << 20, 1 << 20], check_disjoint=True).stats()
+    assert (st.n_device_segments, st.n_chunks) == (segments, chunks)
 
 
 def test_zero_fill_reads_nothing():
