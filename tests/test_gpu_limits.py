@@ -5,6 +5,7 @@
 - Segments beyond 2^30 units, which emrs_plan_create splits so that the
   kernel's unit arithmetic stays in 32 bits: a 1-D and a 2-D byte segment
   of 1.5 GiB each (the element-wise path, where a unit is one byte).
+- Comparisons on either side of the counts at which the base pointers travel another way.
 - 70,000 segments in one plan, with and without the chunk table.
 Expected results come from torch slicing on the device.
 """
@@ -158,6 +159,40 @@ def test_table_bases_every_segment_kind(gpu_device, lanes, buffer_ops):
                 assert np.array_equal(sets[which][j].cpu().numpy(), want[j]), (k, j)
     finally:
         _native.set_tuning()
+
+
+@pytest.mark.parametrize("n", [4, 5, 64, 65])
+def test_compare_finds_differences_over_many_buffers(gpu_device, n):
+    """8, 10, 128 and 130 destination buffers (a small argument block, the large one, a device table):
+    a comparison of every kind of segment finds what was planted in each buffer, as numpy does."""
+    from tests.helpers import compare_numpy
+
+    size = 4096
+    rng = np.random.default_rng(n)
+    t = _kind_table(rng, n, size)
+    srcs_h = [rng.integers(0, 256, size, dtype=np.uint8) for _ in range(n)]
+    dsts_h = _expected(t, srcs_h, n, size)
+    groups, aux_groups = np.arange(n, dtype=np.uint32), np.arange(n, 2 * n, dtype=np.uint32)
+    srcs, dsts = ([torch.from_numpy(h).to(gpu_device) for h in hs] for hs in (srcs_h, dsts_h))
+    plan, fresh = (_native.Plan(t, [size] * n, [size] * (2 * n), check_disjoint=True) for _ in range(2))
+    bases = [s.data_ptr() for s in srcs], [d.data_ptr() for d in dsts]
+    st = torch.cuda.current_stream().cuda_stream
+    print(f"case compare over {n} and {2 * n} buffers", flush=True)
+    for planted in (False, True):
+        if planted:
+            for i, s in enumerate(t):
+                last = int(s["len"]) - 1 + (int(s["rows"]) - 1) * int(s["dst_stride"]) + int(s["dst_off"])
+                dsts_h[i][last * int(s["elem_bytes"])] ^= 1
+                if int(s["flags"]) & 5:
+                    dsts_h[n + i][int(s["aux_off"]) * (2 if int(s["flags"]) & 1 else int(s["elem_bytes"]))] ^= 1
+            for d, h in zip(dsts, dsts_h):
+                d.copy_(torch.from_numpy(h))
+        want = compare_numpy(t, groups, aux_groups, 2 * n, srcs_h, dsts_h)
+        assert bool(want["mismatches"][:n].all()) == planted
+        for p, no_alloc in ((fresh, True), (plan, False), (plan, True)):
+            got = p.compare(*bases, groups, aux_groups, 2 * n, st, no_alloc=no_alloc)
+            assert np.array_equal(got["mismatches"], want["mismatches"]), (planted, no_alloc)
+            assert np.array_equal(got["elements"], want["elements"])
 
 
 def test_segments_beyond_two_to_the_thirty_units(gpu_device):
