@@ -743,16 +743,18 @@ __global__ __launch_bounds__(L) void copy_plan_kernel(const DevSeg *__restrict__
   constexpr uint32_t kPieces = kChunkUnits / (L * U);  // pieces per chunk: 1, 2 or 4
   static_assert(kPieces * L * U == kChunkUnits, "a piece divides a chunk");
   uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
-  if (w < n_warm) {
-    warm_tables<L>(chunk_seg, segs, n_chunks, n_segs, (uint32_t)w);
-    return;
+  if constexpr (kBuf) {  // without buffer instructions, a launch with the chunk table takes copy_pieces_kernel
+    if (w < n_warm) {
+      warm_tables<L>(chunk_seg, segs, n_chunks, n_segs, (uint32_t)w);
+      return;
+    }
+    w -= n_warm;
   }
-  w -= n_warm;
   w = xcd_order(w, xcd_end, xcd_log2);
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;
   uint32_t lo;
-  if (chunk_seg) {  // the segment of every chunk, looked up
+  if (kBuf && chunk_seg) {  // the segment of every chunk, looked up
     lo = chunk_seg[c];
   } else {  // found by a binary search bounded by the hint
     const uint32_t b = (uint32_t)(c >> hint.shift);
