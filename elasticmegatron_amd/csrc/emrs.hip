@@ -380,7 +380,7 @@ __device__ __forceinline__ void copy_chunk_run(const DevSeg *__restrict__ segs, 
     char *db = base_of<kTable>(dst, dst_tab, s.dst_buf());
     char *ab = base_of<kTable>(dst, dst_tab, s.aux_buf());
     const uint32_t ops = s.ops(), ul = s.unit_log2();
-    if (ul == kRowUnits) {
+    if (s.by_rows()) {
 #pragma unroll 1
       for (uint32_t u = u0; u < u_end; u += kThreads * kRowStep)
         dispatch_rows<kNT, kThreads, kRowStep>(s, sb, db, ab, u, u_end);
@@ -603,80 +603,82 @@ __device__ __forceinline__ void copy_units_buf(const DevSeg &s, const char *sbas
   }
 }
 
-template <bool kNT, bool kZero, bool kDup, int L, int U>
-__device__ __forceinline__ void dispatch_chunk_buf(uint32_t ul, const DevSeg &s, const char *sb, char *db,
-                                                   char *ab, uint32_t u0, uint32_t total) {
-  switch (ul) {
-    case 4: copy_units_buf<u32x4, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-    case 3: copy_units_buf<uint64_t, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-    case 2: copy_units_buf<uint32_t, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-    case 1: copy_units_buf<uint16_t, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-    default: copy_units_buf<uint8_t, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
+// One piece by `UnitsOf<T, kCast, kZero, kDup>` for the segment's unit width and what its ops ask for.
+// 16-byte units first, which most segments have: every wave walks these scalar tests, and workgroups
+// of several waves that only store are bound by scalar instructions, of which a CU issues one a cycle.
+// 26 GiB of zeros by workgroups of 256 and 128 lanes: 6.4 and 6.1 TB/s with the ops tested before the
+// unit and the order computed in 64 bits, 7.2 and 7.3 so.
+template <template <typename, bool, bool, bool> class UnitsOf, typename... A>
+__device__ __forceinline__ void dispatch_piece(const DevSeg &s, A... a) {
+  const uint32_t ops = s.ops(), ul = s.unit_log2();
+  if (ul == 4) {
+    switch (ops) {
+      case 0: UnitsOf<u32x4, false, false, false>::run(s, a...); break;
+      case 1: UnitsOf<u32x4, true, false, false>::run(s, a...); break;
+      case 2: UnitsOf<u32x4, false, true, false>::run(s, a...); break;
+      case 3: UnitsOf<u32x4, true, true, false>::run(s, a...); break;
+      case 4: UnitsOf<u32x4, false, false, true>::run(s, a...); break;
+      default: UnitsOf<u32x4, false, true, true>::run(s, a...); break;
+    }
+    return;
+  }
+  if (ops & 1) {  // with the bf16 image: fp32
+    if (ops & 2) UnitsOf<uint32_t, true, true, false>::run(s, a...);
+    else UnitsOf<uint32_t, true, false, false>::run(s, a...);
+    return;
+  }
+  auto elements = [&](auto zero, auto dup) {
+    switch (ul) {
+      case 3: UnitsOf<uint64_t, false, decltype(zero)::value, decltype(dup)::value>::run(s, a...); break;
+      case 2: UnitsOf<uint32_t, false, decltype(zero)::value, decltype(dup)::value>::run(s, a...); break;
+      case 1: UnitsOf<uint16_t, false, decltype(zero)::value, decltype(dup)::value>::run(s, a...); break;
+      default: UnitsOf<uint8_t, false, decltype(zero)::value, decltype(dup)::value>::run(s, a...); break;
+    }
+  };
+  if (ops & 4) {
+    if (ops & 2) elements(std::true_type(), std::true_type());
+    else elements(std::false_type(), std::true_type());
+  } else {
+    if (ops & 2) elements(std::true_type(), std::false_type());
+    else elements(std::false_type(), std::false_type());
   }
 }
-
-template <bool kNT, bool kZero, bool kDup, int L, int U>
-__device__ __forceinline__ void dispatch_chunk(uint32_t ul, const DevSeg &s, const char *sb, char *db, char *ab,
-                                               uint32_t u0, uint32_t total) {
-  switch (ul) {
-    case 4: copy_units<u32x4, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-    case 3: copy_units<uint64_t, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-    case 2: copy_units<uint32_t, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-    case 1: copy_units<uint16_t, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-    default: copy_units<uint8_t, kNT, false, kZero, kDup, L, U>(s, sb, db, ab, u0, total); break;
-  }
-}
+template <bool kNT, int L, int U>
+struct ByAddress {
+  template <typename T, bool kCast, bool kZero, bool kDup>
+  struct Units {
+    __device__ static __forceinline__ void run(const DevSeg &s, const char *sb, char *db, char *ab, uint32_t u0,
+                                               uint32_t total) {
+      copy_units<T, kNT, kCast, kZero, kDup, L, U>(s, sb, db, ab, u0, total);
+    }
+  };
+};
+template <bool kNT, int L, int U>
+struct ByBuffer {
+  template <typename T, bool kCast, bool kZero, bool kDup>
+  struct Units {
+    __device__ static __forceinline__ void run(const DevSeg &s, const char *sb, char *db, char *ab, uint32_t u0,
+                                               uint32_t total) {
+      copy_units_buf<T, kNT, kCast, kZero, kDup, L, U>(s, sb, db, ab, u0, total);
+    }
+  };
+};
 
 // Units [u0, u0 + L * U) of segment s by a workgroup of L lanes.
 template <bool kNT, int L, int U>
 __device__ __forceinline__ void copy_piece(const DevSeg &s, const char *sb, char *db, char *ab, uint32_t u0,
                                            uint32_t total) {
-  const uint32_t ops = s.ops(), ul = s.unit_log2();
-  if (__builtin_expect(ops == 0 && ul == 4, 1)) {  // most of every plan
-    copy_units<u32x4, kNT, false, false, false, L, U>(s, sb, db, ab, u0, total);
-  } else if (ul == kRowUnits) {
-    dispatch_rows<kNT, L, U>(s, sb, db, ab, u0, total);
-  } else if (ops & 4) {  // duplicate to aux, with or without zero fill
-    if (ops & 2) dispatch_chunk<kNT, true, true, L, U>(ul, s, sb, db, ab, u0, total);
-    else dispatch_chunk<kNT, false, true, L, U>(ul, s, sb, db, ab, u0, total);
-  } else if (ops & 1) {  // with the bf16 image (fp32 only: 16- or 4-byte units), with or without zero fill
-    if (ops & 2) {
-      if (ul == 4) copy_units<u32x4, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
-      else copy_units<uint32_t, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
-    } else {
-      if (ul == 4) copy_units<u32x4, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
-      else copy_units<uint32_t, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
-    }
-  } else if (ops & 2) {
-    dispatch_chunk<kNT, true, false, L, U>(ul, s, sb, db, ab, u0, total);
-  } else {
-    dispatch_chunk<kNT, false, false, L, U>(ul, s, sb, db, ab, u0, total);
-  }
+  if (__builtin_expect(s.plain(), 1)) copy_units<u32x4, kNT, false, false, false, L, U>(s, sb, db, ab, u0, total);
+  else if (s.by_rows()) dispatch_rows<kNT, L, U>(s, sb, db, ab, u0, total);
+  else dispatch_piece<ByAddress<kNT, L, U>::template Units>(s, sb, db, ab, u0, total);
 }
 
 // copy_piece with every unit width but row units through buffer instructions.
 template <bool kNT, int L, int U>
 __device__ __forceinline__ void copy_piece_buf(const DevSeg &s, const char *sb, char *db, char *ab, uint32_t u0,
                                                uint32_t total) {
-  const uint32_t ops = s.ops(), ul = s.unit_log2();
-  if (ul == kRowUnits) {
-    dispatch_rows<kNT, L, U>(s, sb, db, ab, u0, total);
-  } else if (ops & 4) {
-    if (ops & 2) dispatch_chunk_buf<kNT, true, true, L, U>(ul, s, sb, db, ab, u0, total);
-    else dispatch_chunk_buf<kNT, false, true, L, U>(ul, s, sb, db, ab, u0, total);
-  } else if (ops & 1) {  // with the bf16 image (fp32 only: 16- or 4-byte units)
-    if (ops & 2) {
-      if (ul == 4) copy_units_buf<u32x4, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
-      else copy_units_buf<uint32_t, kNT, true, true, false, L, U>(s, sb, db, ab, u0, total);
-    } else {
-      if (ul == 4) copy_units_buf<u32x4, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
-      else copy_units_buf<uint32_t, kNT, true, false, false, L, U>(s, sb, db, ab, u0, total);
-    }
-  } else if (ops & 2) {
-    dispatch_chunk_buf<kNT, true, false, L, U>(ul, s, sb, db, ab, u0, total);
-  } else {
-    dispatch_chunk_buf<kNT, false, false, L, U>(ul, s, sb, db, ab, u0, total);
-  }
+  if (s.by_rows()) dispatch_rows<kNT, L, U>(s, sb, db, ab, u0, total);
+  else dispatch_piece<ByBuffer<kNT, L, U>::template Units>(s, sb, db, ab, u0, total);
 }
 
 // A descriptor in one scalar load of 64 bytes.  `p` is uniform over the wave
@@ -744,11 +746,11 @@ __global__ __launch_bounds__(L) void copy_plan_kernel(const DevSeg *__restrict__
   static_assert(kPieces * L * U == kChunkUnits, "a piece divides a chunk");
   uint64_t w = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
   if constexpr (kBuf) {  // without buffer instructions, a launch with the chunk table takes copy_pieces_kernel
-    if (w < n_warm) {
-      warm_tables<L>(chunk_seg, segs, n_chunks, n_segs, (uint32_t)w);
+    w -= n_warm;
+    if ((int32_t)(w >> 32) < 0) {
+      warm_tables<L>(chunk_seg, segs, n_chunks, n_segs, blockIdx.x);
       return;
     }
-    w -= n_warm;
   }
   w = xcd_order(w, xcd_end, xcd_log2);
   const uint64_t c = w / kPieces;
@@ -797,12 +799,11 @@ __global__ __launch_bounds__(L) void copy_pieces_kernel(const uint32_t *__restri
                                                         uint32_t n_segs) {
   constexpr uint32_t kPieces = kChunkUnits / (L * U);  // pieces per chunk: 1, 2 or 4
   static_assert(kPieces * L * U == kChunkUnits, "a piece divides a chunk");
-  uint64_t w = (uint64_t)blockIdx.y * gx + blockIdx.x;
-  if (w < n_warm) {
-    warm_tables<L>(chunk_seg, segs, n_chunks, n_segs, (uint32_t)w);
+  uint64_t w = (uint64_t)blockIdx.y * gx + blockIdx.x - n_warm;
+  if ((int32_t)(w >> 32) < 0) {  // the sign: among the first n_warm
+    warm_tables<L>(chunk_seg, segs, n_chunks, n_segs, blockIdx.x);
     return;
   }
-  w -= n_warm;
   w = xcd_order(w, xcd_end, xcd_log2);
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;
@@ -1712,12 +1713,11 @@ __global__ __launch_bounds__(64) void differ_piece_kernel(
     uint32_t gx, uint32_t n_warm, uint32_t xcd_log2, const uint64_t *__restrict__ src_tab, const uint64_t *__restrict__ dst_tab, B src,
     B dst, uint32_t n_segs, DifferMarks marks) {
   constexpr uint32_t kPieces = kChunkUnits / (64 * U);
-  uint64_t w = (uint64_t)blockIdx.y * gx + blockIdx.x;
-  if (w < n_warm) {
-    warm_tables<64>(chunk_seg, segs, n_chunks, n_segs, (uint32_t)w);
+  uint64_t w = (uint64_t)blockIdx.y * gx + blockIdx.x - n_warm;
+  if ((int32_t)(w >> 32) < 0) {  // the sign: among the first n_warm
+    warm_tables<64>(chunk_seg, segs, n_chunks, n_segs, blockIdx.x);
     return;
   }
-  w -= n_warm;
   w = xcd_order(w, xcd_end, xcd_log2);
   const uint64_t c = w / kPieces;
   if (c >= n_chunks) return;

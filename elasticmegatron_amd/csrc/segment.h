@@ -61,7 +61,7 @@ struct DevSeg {
   uint32_t meta;         // bits 0-15: second destination (aux) buffer; 16-23: shifts; 24-31: kind
 
   // shifts: bits 0-4 sh2, bit 5 sh1, bit 6 row units on lines (else on 16-byte
-  // boundaries).  kind: bits 0-2 unit_log2 (or kRowUnits), bits 3-4
+  // boundaries), bit 7 row units (again: one bit to test).  kind: bits 0-2 unit_log2 (or kRowUnits), bits 3-4
   // elem_log2, bits 5-7 ops.  ops bit 0: also write bf16 to aux; bit 1: write
   // zeros, read nothing; bit 2: also write the values unchanged to aux.
   // elem_log2: element size of the input segment (read by the compare kernel
@@ -74,6 +74,9 @@ struct DevSeg {
   EMRS_HD uint32_t unit_log2() const { return (meta >> 24) & 7u; }
   EMRS_HD uint32_t elem_log2() const { return (meta >> 27) & 3u; }
   EMRS_HD uint32_t ops() const { return meta >> 29; }
+  EMRS_HD bool by_rows() const { return (meta >> 23) & 1u; }
+  // A copy of 16-byte units with one destination: most of every plan.
+  EMRS_HD bool plain() const { return (meta & 0xe7000000u) == 4u << 24; }
   void set_bufs(uint32_t src, uint32_t dst, uint32_t aux) {
     bufs = (src & 0xffffu) | (dst << 16);
     meta = (meta & 0xffff0000u) | (aux & 0xffffu);
@@ -82,15 +85,15 @@ struct DevSeg {
   EMRS_HD uint32_t phase_mask() const { return (meta >> 22) & 1u ? 127u : 15u; }
   // Units in a row, and in the segment.
   EMRS_HD uint32_t row_units() const {
-    if (unit_log2() != kRowUnits) return len;
+    if (!by_rows()) return len;
     const uint32_t lg = elem_log2();
     return (len + (phase_mask() >> lg) + (15u >> lg)) >> (4 - lg);
   }
   EMRS_HD uint32_t units() const { return row_units() * rows; }
   // log2 of the bytes that offsets and strides count.
-  EMRS_HD uint32_t off_log2() const { return unit_log2() == kRowUnits ? elem_log2() : unit_log2(); }
+  EMRS_HD uint32_t off_log2() const { return by_rows() ? elem_log2() : unit_log2(); }
   void set_kind(uint32_t unit_log2_, uint32_t elem_log2_, uint32_t ops_, bool on_lines) {
-    meta = (meta & 0x003fffffu) | ((on_lines ? 1u : 0u) << 22) |
+    meta = (meta & 0x003fffffu) | ((on_lines ? 1u : 0u) << 22) | ((unit_log2_ == kRowUnits ? 1u : 0u) << 23) |
            ((unit_log2_ | (elem_log2_ << 3) | (ops_ << 5)) << 24);
   }
   void set_division(uint32_t magic_, uint32_t sh1_, uint32_t sh2_) {
@@ -158,9 +161,9 @@ constexpr uint32_t kXcdEighths = 63;  // in place of a run's log2, see xcd_order
 // neighbours share, and its translation caches fewer pages.
 EMRS_HD inline uint64_t xcd_order(uint64_t w, uint64_t end, uint32_t lg) {
   if (w >= end) return w;
-  if (lg == kXcdEighths) return (w & 7) * (end >> 3) + (w >> 3);
-  const uint64_t i = w & ((8ull << lg) - 1);
-  return w - i + ((i & 7) << lg) + (i >> 3);
+  if (__builtin_expect(lg == kXcdEighths, 0)) return (w & 7) * (end >> 3) + (w >> 3);
+  const uint32_t mask = (8u << lg) - 1, i = (uint32_t)w & mask;  // the low lg + 3 bits rotate
+  return (w & ~(uint64_t)mask) | ((i & 7) << lg) | (i >> 3);
 }
 
 // Chunks in a run of one XCD (see xcd_order): 2^8 (1 MB of 16-byte units), and

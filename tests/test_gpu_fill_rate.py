@@ -1,0 +1,51 @@
+"""GPU: what a workgroup of several waves costs beyond its stores.
+
+Every wave of a workgroup walks the same scalar instructions before it stores.  Filling with zeros,
+nothing is waited for, so that workgroups of 128 and 256 lanes run at the memory's rate only while
+those instructions are few; workgroups of one wave are bound by the rate of launching workgroups.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from elasticmegatron_amd import _native
+from elasticmegatron_amd.resharding.layout import SEGMENT_DTYPE
+
+pytestmark = pytest.mark.gpu
+
+
+def test_zero_fill_in_larger_workgroups_runs_at_the_memorys_rate(gpu_device):
+    """Measured on 26 GiB: 4.85 TB/s with 64 lanes of one unit; 7.2 and 7.3 with 256 and 128, where 105
+    scalar instructions a wave in place of about 75 gave 6.4 and 6.1."""
+    nbytes = 16 << 30
+    dst = torch.empty(nbytes // 4, dtype=torch.int32, device=gpu_device)
+    t = np.zeros(1, dtype=SEGMENT_DTYPE)
+    t[0] = (0, 0, 4, 2, 0, 0, nbytes // 4, 1, 0, 0, 0, 0, 0, 0)
+    plan = _native.Plan(t, [16], [nbytes])
+    st = torch.cuda.current_stream().cuda_stream
+
+    def best_ms():
+        plan.execute([dst.data_ptr()], [dst.data_ptr()], st)
+        times = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(3):
+                plan.execute([dst.data_ptr()], [dst.data_ptr()], st)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b) / 3)
+        return min(times)
+
+    ms = {}
+    try:
+        for lanes in (64, 128, 256):
+            dst.fill_(1)
+            _native.set_tuning(lanes=lanes, units=1)
+            ms[lanes] = best_ms()
+            assert not dst.any(), lanes
+    finally:
+        _native.set_tuning()
+    print("TB/s by lanes:", {k: round(nbytes / v / 1e9, 2) for k, v in ms.items()}, flush=True)
+    assert ms[64] / ms[128] > 1.4 and ms[64] / ms[256] > 1.4, ms
