@@ -1939,6 +1939,19 @@ __global__ void clear_words_kernel(uint32_t *p, uint64_t n) {
     p[i] = 0;
 }
 
+// The groups that a first pass's flags mark, into `active` (all zero before); leaves the flags zero.
+__global__ void mark_groups_kernel(uint32_t *__restrict__ flags, const uint32_t *__restrict__ groups,
+                                   const uint32_t *__restrict__ aux_groups, uint32_t n_segs,
+                                   uint8_t *__restrict__ active) {
+  for (uint64_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n_segs; k += gridDim.x * blockDim.x) {
+    const uint32_t f = flags[k];
+    if (!f) continue;
+    if (f & 1u) active[groups[k]] = 1;
+    if (f & 2u) active[aux_groups[k]] = 1;
+    flags[k] = 0;
+  }
+}
+
 // A grid of `n_wg` workgroups of `lanes` lanes, with fewer than 8 more per row:
 // one row up to the 2^32 - 1 lanes that a dimension holds, else as many equal
 // rows as that takes, each a multiple of 8 workgroups long so that a
@@ -2096,14 +2109,17 @@ hipError_t clear_words(void *p, uint64_t words, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Second pass of a comparison, when the first has marked groups: every figure
-// of those, on device buffers the caller provides (acc: n_groups accumulators;
-// grp: two group ids per device segment; active: n_groups bytes), leaving the
-// accumulators in `host`.  Waits for the stream: `mark` and the group table
-// are read by the copies.
+// Second pass of a comparison, when the first has marked segments: every figure
+// of their groups, on device buffers the caller provides (acc: n_groups
+// accumulators; grp: two group ids per device segment; active: n_groups bytes,
+// in whole words), leaving the accumulators in `host`.  The groups are those of
+// `mark` or, where it is null, those that `flags` mark on the device, which are
+// zero afterwards: read back to the host, they cost a comparison that finds
+// something one more wait (4 KB 57 us, and 76 with the wait; 240 MB in 60,000
+// segments 489 and 553).  Waits for the stream: `mark` and the group table are read by the copies.
 hipError_t compare_marked(const emrs_plan *plan, const CompareJob &job, const DevSeg *table, uint32_t *grp,
-                          const uint64_t *tab, GroupAcc *acc, uint8_t *active, const std::vector<uint8_t> &mark,
-                          hipStream_t st, std::vector<GroupAcc> &host) {
+                          const uint64_t *tab, GroupAcc *acc, uint8_t *active, const std::vector<uint8_t> *mark,
+                          uint32_t *flags, hipStream_t st, std::vector<GroupAcc> &host) {
   const uint32_t nd = (uint32_t)plan->segs.size();
   const uint64_t *dtab = tab ? tab + plan->stats.n_src_bufs : nullptr;
   const std::vector<uint32_t> gt = job.group_table(plan);
@@ -2111,7 +2127,16 @@ hipError_t compare_marked(const emrs_plan *plan, const CompareJob &job, const De
   uint32_t run = 0;
   persistent_grid(plan, job, resident_of(compare_plan_kernel<false>), &grid, &run);
   hipError_t e = hipMemcpyAsync(grp, gt.data(), gt.size() * sizeof(uint32_t), hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(active, mark.data(), mark.size(), hipMemcpyHostToDevice, st);
+  if (mark) {
+    if (e == hipSuccess) e = hipMemcpyAsync(active, mark->data(), mark->size(), hipMemcpyHostToDevice, st);
+  } else {
+    if (e == hipSuccess) e = clear_words(active, (host.size() + 3) / 4, st);
+    if (e == hipSuccess) {
+      hipLaunchKernelGGL(mark_groups_kernel, dim3(std::min<uint32_t>(1024, (nd + 255) / 256)), dim3(256), 0, st, flags,
+                         grp, grp + nd, nd, active);
+      e = hipGetLastError();
+    }
+  }
   if (e == hipSuccess) e = clear_words(acc, host.size() * sizeof(GroupAcc) / sizeof(uint32_t), st);
   if (e == hipSuccess) {
     if (job.rb.table)
@@ -2633,30 +2658,30 @@ int emrs_plan_compare(emrs_plan *plan, void *const *src_bases, void *const *dst_
   hipError_t e = differ_launch(plan, job, table, tab, DifferMarks{flags, any}, st);
   const hipError_t se = hipStreamSynchronize(st);
   if (e == hipSuccess) e = se;
-  const bool marked = any == nullptr || *static_cast<volatile uint32_t *>(any) != 0;
+  const bool differs = any && *static_cast<volatile uint32_t *>(any) != 0;
   give_any_slot(any);
   std::vector<GroupAcc> host(n_groups);
-  bool clean = e == hipSuccess;
-  if (e == hipSuccess && marked) {
+  bool clean = e == hipSuccess, marked = differs;
+  if (e == hipSuccess && !any) {  // no word was set: the flags themselves tell
     std::vector<uint32_t> found(nd);
-    std::vector<uint8_t> mark(n_groups, 0);
-    clean = false;
     e = hipMemcpyAsync(found.data(), flags, nd * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = clear_words(flags, nd, st);
     const hipError_t fe = hipStreamSynchronize(st);
     if (e == hipSuccess) e = fe;
     clean = e == hipSuccess;
-    if (e == hipSuccess && job.marked_groups(plan, found, &mark)) {
-      const size_t acc_bytes = align256((size_t)n_groups * sizeof(GroupAcc));
-      const size_t grp_bytes = align256(2 * nd * sizeof(uint32_t));
-      char *buf = nullptr;
-      e = hipMalloc(&buf, acc_bytes + grp_bytes + n_groups);
-      if (e == hipSuccess) {
-        e = compare_marked(plan, job, table, reinterpret_cast<uint32_t *>(buf + acc_bytes), tab,
-                           reinterpret_cast<GroupAcc *>(buf), reinterpret_cast<uint8_t *>(buf + acc_bytes + grp_bytes),
-                           mark, st, host);
-        (void)hipFree(buf);
-      }
+    marked = std::any_of(found.begin(), found.end(), [](uint32_t f) { return f != 0; });
+  }
+  if (e == hipSuccess && marked) {
+    clean = false;
+    const size_t acc_bytes = align256((size_t)n_groups * sizeof(GroupAcc));
+    const size_t grp_bytes = align256(2 * nd * sizeof(uint32_t));
+    char *buf = nullptr;
+    e = hipMalloc(&buf, acc_bytes + grp_bytes + align256(n_groups));
+    if (e == hipSuccess) {
+      e = compare_marked(plan, job, table, reinterpret_cast<uint32_t *>(buf + acc_bytes), tab,
+                         reinterpret_cast<GroupAcc *>(buf), reinterpret_cast<uint8_t *>(buf + acc_bytes + grp_bytes),
+                         nullptr, flags, st, host);
+      (void)hipFree(buf);
+      clean = e == hipSuccess;
     }
   }
   give_flags(plan, dev, st, flags, clean);
@@ -2720,7 +2745,7 @@ int emrs_plan_compare_static(emrs_plan *plan, void *const *src_bases, void *cons
   if (e == hipSuccess) e = hipMemcpyAsync(found.data(), grp, nd * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e == hipSuccess && job.marked_groups(plan, found, &mark))
-    e = compare_marked(plan, job, table, grp, tab, acc, active, mark, st, host);
+    e = compare_marked(plan, job, table, grp, tab, acc, active, &mark, nullptr, st, host);
   // The host copies above read job's and plan's vectors: wait before they can go.
   const hipError_t se = hipStreamSynchronize(st);
   if (e == hipSuccess) e = se;

@@ -283,3 +283,38 @@ def test_more_than_65535_segments(gpu_device, chunk_index):
     want = src.view(n, unit)[perm.to(gpu_device)].clone()
     want[torch.from_numpy(zero).to(gpu_device)] = 0
     assert torch.equal(dst.view(n, unit), want)
+
+
+def test_groups_of_marked_segments_beyond_one_grid(gpu_device):
+    """300,000 duplicating segments, more than one pass of the grid that marks their groups, and 13 groups,
+    no whole number of words: only the groups of the three segments that differ report anything."""
+    n, w = 300_000, 4
+    t = np.zeros(n, dtype=SEGMENT_DTYPE)
+    k = np.arange(n, dtype=np.uint64)
+    t["elem_bytes"], t["flags"], t["len"], t["rows"], t["aux_buf"] = 4, 4, w, 1, 1
+    t["src_off"] = t["dst_off"] = t["aux_off"] = k * w
+    src = torch.arange(n * w, dtype=torch.int32, device=gpu_device)
+    dst, aux = torch.zeros_like(src), torch.zeros_like(src)
+    plan = _native.Plan(t, [n * w * 4], [n * w * 4] * 2)
+    groups, aux_groups = (k % 7).astype(np.uint32), (7 + k % 6).astype(np.uint32)
+    st = torch.cuda.current_stream().cuda_stream
+    bases = [src.data_ptr()], [dst.data_ptr(), aux.data_ptr()]
+    plan.execute(*bases, st)
+
+    def compare():
+        return plan.compare(*bases, groups, aux_groups, 13, st)["mismatches"].astype(int).tolist()
+
+    print("case 300000 segments in 13 groups", flush=True)
+    assert compare() == [0] * 13
+    dst[0] ^= 1
+    dst[(n - 2) * w + 3] ^= 1
+    aux[(n - 1) * w] ^= 1
+    want = [0] * 13
+    want[0] += 1
+    want[(n - 2) % 7] += 1
+    want[7 + (n - 1) % 6] += 1
+    assert compare() == want and compare() == want
+    dst[0] ^= 1
+    dst[(n - 2) * w + 3] ^= 1
+    aux[(n - 1) * w] ^= 1
+    assert compare() == [0] * 13
