@@ -1446,7 +1446,7 @@ def copy_ceiling(a, b, stream, traffic_gbps, read_bytes, write_bytes, reps=5):
     """What the very allocations the reshard ran on can do (physical placement moves every figure
     together), with the same 16-byte non-temporal accesses:
 
-    - a plain contiguous copy of the source main arena into the destination one, by copy_plan_kernel;
+    - a plain contiguous copy of the source main arena into the destination one, by the copy kernel;
     - write-only: the same kernel zero-filling the destination main arena (no reads), with one
       workgroup per 4 KB chunk whatever the launch shape (a workgroup that only stores 1 KB is so
       short that the rate of launching workgroups, not the memory, would bound the figure), in the
@@ -1512,7 +1512,7 @@ def copy_ceiling(a, b, stream, traffic_gbps, read_bytes, write_bytes, reps=5):
     w_gbps, r_gbps = n * 4 / (w_ms / 1e3) / 1e9, n * 4 / (r_ms / 1e3) / 1e9
     serial = (read_bytes + write_bytes) / (read_bytes / r_gbps + write_bytes / w_gbps)
     return {"gbps": round(gbps, 1), "bytes_per_launch": 2 * n * 4, "ms": round(ms, 4),
-            "what": "one contiguous copy of the main arena by copy_plan_kernel, same allocations",
+            "what": f"one contiguous copy of the main arena by {copy_kernel()}, same allocations",
             "reshard_frac_of_copy": round(traffic_gbps / gbps, 4),
             "read_only_gbps": round(r_gbps, 1), "write_only_gbps": round(w_gbps, 1),
             "write_only_gbps_by_shape": {k: round(n * 4 / (v / 1e3) / 1e9, 1) for k, v in w_shapes.items()},

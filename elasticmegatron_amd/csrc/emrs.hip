@@ -2,14 +2,15 @@
 //
 // One launch moves every segment of a plan.  The path is pure data movement
 // (no arithmetic), so the kernel is shaped for HBM streaming: the plan is cut
-// into chunks of 256 units (4 KB of 16-byte units), and every chunk is a
-// workgroup of its own, one wave of 64 lanes with four units each, that finds
-// its segment by one binary search, issues its four loads, stores and exits.
-// The hardware dispatches workgroups in order, so the in-flight ones always
-// cover one narrow window of the plan that sweeps through memory; a
-// persistent grid, whose workgroups drift apart, writes up to 20% slower on
-// most physical placements of the same buffers.  The persistent grid remains
-// as a tuning option.  Element sizes are irrelevant to the vector path:
+// into chunks of 256 units (4 KB of 16-byte units), and every chunk into four
+// pieces, each a workgroup of its own: one wave of 64 lanes with one unit each
+// that reads its segment's number from the plan's chunk table and the segment's
+// descriptor, loads, stores and exits.  The hardware dispatches workgroups in
+// order, so the in-flight ones always cover a few narrow windows of the plan (a
+// run of chunks for each XCD) that sweep through memory; a persistent grid,
+// whose workgroups drift apart, writes up to 20% slower on most physical
+// placements of the same buffers.  The persistent grid remains as a tuning
+// option.  Element sizes are irrelevant to the vector path:
 // offsets are converted to 16-byte units when the plan is created, so bf16
 // parameters and fp32 optimizer state share one launch.
 //
@@ -1665,7 +1666,8 @@ __device__ __forceinline__ void mark_segment(const DifferMarks &m, uint32_t seg,
 }
 
 // The bit-level pass over row units [u0, u0 + L * U) (clipped to u_end), every
-// load issued before the comparison.  Elements that two units hold are looked at twice.
+// load of the source and the destination issued before the comparison, the second destination's after
+// it.  Elements that two units hold are looked at twice.
 template <int L, int U>
 __device__ __forceinline__ void differ_rows(const DevSeg &s, const char *sbase, const char *dbase, const char *abase,
                                             uint32_t u0, uint32_t u_end, uint32_t &dm, uint32_t &dx) {
@@ -1699,8 +1701,8 @@ __device__ __forceinline__ void differ_rows(const DevSeg &s, const char *sbase, 
 // First pass of a comparison on the copy kernel's schedule and with its short
 // chain of scalar loads (see copy_pieces_kernel): the first workgroups read the
 // tables, then one 64-lane workgroup per piece of U units a lane takes its
-// segment from the plan's chunk table, dispatched in order and, on large plans,
-// XCDs in runs (xcd_order).  Faster than the persistent grid on
+// segment from the plan's chunk table, dispatched in order, the XCDs in runs
+// (xcd_order).  Faster than the persistent grid on
 // every full-size switch (2-4%, same allocations): a segment's rows or gathered
 // runs are spread over many workgroups in flight.  Bound by reading HBM.  Whole
 // calls before the pre-read, the preloaded arguments, two units a lane and the

@@ -446,10 +446,10 @@ def _assemble(fp32: np.ndarray, bf16: np.ndarray, g32: np.ndarray, gbf: np.ndarr
     A duplicating segment duplicates within its own kind's arena.
 
     The kinds are interleaved segment by segment, in pieces of at most
-    64 MiB: a main chunk that also writes the bf16 cast costs more than the
-    others, and each XCD sweeps its own eighth of the plan, so every eighth
-    must hold the same mix of kinds.  Running the kinds one after another
-    instead costs 8% on Llama-2-7B.
+    64 MiB: a main chunk that also writes the bf16 cast moves more than the
+    others, so kinds one after another change the mix of reads and writes over
+    the launch, and, where each XCD sweeps an eighth of the plan, leave some
+    XCDs more to do than others.  With such eighths it cost 8% on Llama-2-7B.
     """
     base, gbase = _split(fp32, INTERLEAVE_ELEMS, g32)
     out = np.zeros(3 * len(base), dtype=SEGMENT_DTYPE)

@@ -230,9 +230,9 @@ typedef struct emrs_compare_stats {
 /*
  * Compare the destination buffers with what `plan` writes from the source
  * buffers, and accumulate the differences per group.  Two passes: the first
- * only finds the groups in which any bit differs, at the rate of a plain read;
- * only if there are such groups does a second pass compute every figure for
- * them.  A correct switch therefore costs one read of the source and the
+ * only finds the segments in which any bit differs, at the rate of a plain read;
+ * only if there are such segments does a second pass compute every figure for
+ * their groups.  A correct switch therefore costs one read of the source and the
  * destination.
  *   groups[i]:     group of input segment i's elements (NULL: all group 0)
  *   aux_groups[i]: group of input segment i's bf16 image (NULL: groups[i])
@@ -240,9 +240,14 @@ typedef struct emrs_compare_stats {
  * Base pointers follow emrs_plan_execute's rules, except that buffers may
  * overlap: a comparison only reads (a state that took over part of its
  * source's memory compares equal there).  The call runs on `stream`
- * and waits for it.  It allocates and frees a small device buffer (the
- * group tables and accumulators), so it is not for capture into a graph:
- * while `stream` is capturing it returns EMRS_ERR_CAPTURE.
+ * and waits for it.  The first call on a device uploads the plan's tables as
+ * emrs_plan_execute does, and allocates the first pass's marks (4 bytes per
+ * device segment), which the plan keeps until it is destroyed; the process's
+ * first comparison also allocates a page of pinned host memory that every
+ * comparison is told a difference through.  A call that finds a difference
+ * allocates and frees a device buffer for the group tables and accumulators.
+ * So it is not for capture into a graph: while `stream` is capturing it
+ * returns EMRS_ERR_CAPTURE.
  * Errors: INVALID_ARGUMENT (n_groups == 0, a group id >= n_groups), the
  * base-pointer errors of emrs_plan_execute but ALIAS, CAPTURE, NO_DEVICE, HIP.
  */
@@ -262,7 +267,8 @@ int emrs_plan_compare(emrs_plan *plan, void *const *src_bases, void *const *dst_
  * process ends.  A comparison that needs more (about 50,000 device segments
  * with few groups) returns EMRS_ERR_TOO_LARGE and does nothing.  The array is
  * shared by every call on a device and keeps the last call's contents; the
- * accumulators are cleared at the start of each call.  The library serialises
+ * marks are cleared at the start of each call, and the accumulators before the
+ * second pass, in calls that run one.  The library serialises
  * the calls of one process on one device, and each call waits for `stream`
  * before it returns, so calls never overlap in their use of the array.  Not
  * for capture into a graph (EMRS_ERR_CAPTURE).
