@@ -176,8 +176,14 @@ EMRS_HD inline uint64_t xcd_order(uint64_t w, uint64_t end, uint32_t lg) {
 // 164.6, 155.8, 155.4, 155.8; 1.02 GB of long runs 163.0, 170.1, 164.6, 167.9;
 // 2.66 GB of short rows 481, 436, 431, 436; 3.4 GB Group ZeRO 637, 605, 595, 597;
 // (eighths, 2^8, 2^10) 9.2 GB of short rows 1480, 1475, 1472; 28 GB 4303, 4339,
-// 4290; 42 GB 6334, 6374, 6313; 70 GB 10660, 10703, 10678.  Runs of 2^4 were 8-13%
-// slower on the large ones.
+// 4290; 42 GB 6334, 6374, 6313; 70 GB 10660, 10703, 10678.  Runs of 2^4 on plans
+// of every size: 9 GB in short rows 9% slower, 28 GB 11%, 45 GB 6%, 70 GB 4%.
+// Time in runs over time in the hardware's order, 109 plans of 0.04 to 6 GB under
+// 2^19 chunks: 0.85 to 1.00, on average 0.95, where an eighth or more of the bytes
+// lies off 128-byte lines on either side (30 plans); 0.96 to 1.03, on average 1.00,
+// where less does (Group ZeRO to two instances at either end).  Neither the rows'
+// length nor a second destination tells which of those gain, so they take runs too.
+// A comparison's first pass gained on all of the 42 plans it was timed on: 0.92 to 0.99.
 constexpr uint32_t kXcdRunLog2 = 8;
 constexpr uint32_t kXcdLongRunLog2 = 10;
 constexpr uint64_t kXcdLongRunMinChunks = 1ull << 19;
