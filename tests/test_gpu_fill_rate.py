@@ -48,4 +48,6 @@ def test_zero_fill_in_larger_workgroups_runs_at_the_memorys_rate(gpu_device):
     finally:
         _native.set_tuning()
     print("TB/s by lanes:", {k: round(nbytes / v / 1e9, 2) for k, v in ms.items()}, flush=True)
-    assert ms[64] / ms[128] > 1.4 and ms[64] / ms[256] > 1.4, ms
+    # 1.45 to 1.51 as measured, 1.26 and 1.32 with the instructions of before; the memory's own rate moves
+    # by several percent with the placement of the buffer.
+    assert ms[64] / ms[128] > 1.35 and ms[64] / ms[256] > 1.35, ms
